@@ -127,19 +127,20 @@ __device__ __forceinline__ int vswz(int r) {
 // does not treat the in-flight loads as possibly aliasing the other buffer's
 // LDS reads (it otherwise waits for them before some transposing reads); the
 // kernel waits for them itself (vmcnt(0) before the barrier that publishes
-// the tile).  `lds` must be wave-uniform.
-__device__ __forceinline__ void load_lds16(const void* src, const char* lds) {
-  const uint32_t m0 = __builtin_amdgcn_readfirstlane(
-      static_cast<uint32_t>(reinterpret_cast<uintptr_t>(lds)));
-  asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(m0), "v"(src)
+// the tile).  `lds`, the LDS byte address, must be wave-uniform; the s_nop is the wait
+// state between a scalar write of m0 and a load to LDS.
+__device__ __forceinline__ void load_lds16(const void* src, uint32_t lds) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(lds), "v"(src)
                : "memory", "m0");
 }
 // The same from a wave-uniform base address plus a 32-bit per-lane byte offset.
-__device__ __forceinline__ void load_lds16(const void* base, uint32_t voff, const char* lds) {
-  const uint32_t m0 = __builtin_amdgcn_readfirstlane(
-      static_cast<uint32_t>(reinterpret_cast<uintptr_t>(lds)));
-  asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(m0), "v"(voff), "s"(base)
+__device__ __forceinline__ void load_lds16(const void* base, uint32_t voff, uint32_t lds) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds), "v"(voff), "s"(base)
                : "memory", "m0");
+}
+// LDS byte address of a shared object (what m0 of a direct load holds).
+__device__ __forceinline__ uint32_t lds_addr(const char* p) {
+  return __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(reinterpret_cast<uintptr_t>(p)));
 }
 
 // K/V addressing of a kernel instance.
@@ -212,7 +213,7 @@ __global__ __launch_bounds__(kPfThreads, 2) void paged_prefill_attn(PrefillParam
   const int kt0 = klo & ~(kPfKeys - 1);
   const int ntiles = khi >= klo ? (khi - kt0) / kPfKeys + 1 : 0;
 
-  const int wave = threadIdx.x >> 6;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int lane = threadIdx.x & 63;
   const int64_t q0 = kPrefix ? 0 : p.cu_seqlens_q[b];
   const int rows_used = p.tokens_per_wg * G;
@@ -236,13 +237,9 @@ __global__ __launch_bounds__(kPfThreads, 2) void paged_prefill_attn(PrefillParam
     hi_r = valid ? khi : -1;
     lo_r = valid && W >= 0 ? L - 1 - W : 0;
   }
-  // Key range of the wave's valid rows (wave-uniform) for skipping tiles.
+  // Whether the wave has rows at all.
   const int wr0 = wave * 32;
-  const int wt_first = t0 + wr0 / G;
-  const int wt_last = min(t1 - 1, t0 + min(wr0 + 31, rows_used - 1) / G);
-  const bool wave_active = wr0 < rows_used && wt_first < t1;
-  const int wave_hi = kPrefix ? khi : min(Lk - 1, wt_last + off);
-  const int wave_lo = kPrefix ? 0 : (W >= 0 ? wt_first + off - W : 0);
+  const bool wave_active = wr0 < rows_used && t0 + wr0 / G < t1;
 
   // Queries (B operand of S^T, 16 dims per k-step).  A negative scale is
   // applied as a sign flip of q (exact) and |scale|, so the running maxima can
@@ -258,72 +255,101 @@ __global__ __launch_bounds__(kPfThreads, 2) void paged_prefill_attn(PrefillParam
   const int64_t row_stride = static_cast<int64_t>(p.num_kv_heads) * D;
   const uint16_t* kbase = static_cast<const uint16_t*>(p.k) + kh * D;
   const uint16_t* vbase = static_cast<const uint16_t*>(p.v) + kh * D;
-  const int32_t* bt = p.block_table + (MODE == kContiguous ? 0 : b * p.max_blocks);
   const int64_t kstart = p.cu_seqlens_k[b];
+  // Block table read through the constant address space (scalar loads, one per page).
+  typedef __attribute__((address_space(4))) const int32_t bt_t;
+  bt_t* bt = (bt_t*)(p.block_table + (MODE == kContiguous ? 0 : b * p.max_blocks));
   // Per-lane constants: tile row of each load, its byte offset in the tile's
   // source rows, and the swizzled source chunks.
+  const uint32_t strideb = static_cast<uint32_t>(row_stride * 2);
   int trow[NLD];
-  uint32_t koff[NLD], voff[NLD], kchb[NLD], vchb[NLD];
-  int blk_next[NLD];
+  uint32_t rowb[NLD], kchb[NLD], vchb[NLD];
+  int blk_row[NLD];  // kPagedRows: the next tile's block ids
 #pragma unroll
   for (int x = 0; x < NLD; ++x) {
     trow[x] = wave * WROWS + x * RPI + lrow;
     kchb[x] = 16 * (lpos ^ kswz<D>(trow[x]));
     vchb[x] = 32 * ((lpos >> 1) ^ vswz<D>(trow[x])) + 16 * (lpos & 1);
-    koff[x] = static_cast<uint32_t>(trow[x] * row_stride * 2) + kchb[x];
-    voff[x] = static_cast<uint32_t>(trow[x] * row_stride * 2) + vchb[x];
-    blk_next[x] = 0;
+    rowb[x] = static_cast<uint32_t>(trow[x]) * strideb;
+    blk_row[x] = 0;
   }
-  // Block-table entries of the tile at kb0 (one per tile, or one per row),
-  // read a tile ahead of its loads so their latency hides behind a tile of math.
-  auto fetch_blocks = [&](int kb0) {
-    if (MODE == kPagedTiles) {
-      blk_next[0] = bt[kb0 / p.block_size];
-    } else if (MODE == kPagedRows) {
+  // The tile being fetched (tiles are fetched in order): its first key, and for
+  // kPagedTiles its page, the offset inside it, that page's block and the next one's.
+  int f_kb = kt0;
+  int f_in = 0, f_page = 0, f_blk = 0, f_next = 0;
+  const int last_page = ntiles > 0 ? khi / p.block_size : 0;
+  if (MODE == kPagedTiles && ntiles > 0) {
+    f_page = kt0 / p.block_size;
+    f_in = kt0 % p.block_size;
+    f_blk = bt[f_page];
+    f_next = bt[min(f_page + 1, last_page)];
+  }
+  // kPagedRows: block ids of the tile at f_kb, read a tile ahead of its loads.
+  auto fetch_rows = [&]() {
+    if (MODE == kPagedRows) {
 #pragma unroll
-      for (int x = 0; x < NLD; ++x) blk_next[x] = bt[min(kb0 + trow[x], Lk - 1) / p.block_size];
+      for (int x = 0; x < NLD; ++x) blk_row[x] = p.block_table[b * p.max_blocks + min(f_kb + trow[x], Lk - 1) / p.block_size];
     }
   };
-  auto issue_tile = [&](int kb0, char* sbuf) {
+  // Wave-uniform source of the tile at f_kb: base rows and the byte offset of its
+  // last valid row (rows past it repeat it).
+  const uint16_t* f_k = kbase;
+  const uint16_t* f_v = vbase;
+  uint32_t f_limb = 0;
+  auto locate_tile = [&]() {
+    if (MODE == kPagedRows) return;
+    int64_t row0;
+    int lim;
+    if (MODE == kPagedTiles) {
+      row0 = static_cast<int64_t>(min(max(f_blk, 0), p.num_blocks - 1)) * p.block_size + f_in;
+      lim = Lk - 1 - f_kb;
+    } else {
+      row0 = min(kstart + f_kb, p.num_rows - 1);
+      lim = static_cast<int>(min<int64_t>(Lk - 1 - f_kb, p.num_rows - 1 - row0));
+    }
+    f_limb = static_cast<uint32_t>(min(lim, kPfKeys - 1)) * strideb;
+    f_k = kbase + row0 * row_stride;
+    f_v = vbase + row0 * row_stride;
+  };
+  // Load x of the 2 NLD loads of the located tile (K, V alternating).
+  auto issue_load = [&](int x2, uint32_t sbuf) {
+    const int x = x2 >> 1;
+    const uint32_t dst = sbuf + (wave * WROWS + x * RPI) * ROWB + (x2 & 1) * TBYTES;
     if (MODE == kPagedRows) {
       // General pages: a 64-bit source address per lane.
-      int64_t rows[NLD];
-#pragma unroll
-      for (int x = 0; x < NLD; ++x) {
-        const int key = min(kb0 + trow[x], Lk - 1);
-        const int blk = min(max(blk_next[x], 0), p.num_blocks - 1);
-        rows[x] = static_cast<int64_t>(blk) * p.block_size + key % p.block_size;
-      }
-#pragma unroll
-      for (int x = 0; x < NLD; ++x) {
-        char* dst = sbuf + (wave * WROWS + x * RPI) * ROWB;
-        load_lds16(kbase + rows[x] * row_stride + kchb[x] / 2, dst);
-        load_lds16(vbase + rows[x] * row_stride + vchb[x] / 2, dst + TBYTES);
-      }
+      const int key = min(f_kb + trow[x], Lk - 1);
+      const int blk = min(max(blk_row[x], 0), p.num_blocks - 1);
+      const int64_t row = static_cast<int64_t>(blk) * p.block_size + key % p.block_size;
+      if (x2 & 1)
+        load_lds16(vbase + row * row_stride + vchb[x] / 2, dst);
+      else
+        load_lds16(kbase + row * row_stride + kchb[x] / 2, dst);
     } else {
-      // The tile's rows are consecutive: a uniform base row plus per-lane
-      // offsets; rows past the last valid one repeat it.
-      int64_t row0;
-      int lim;  // last valid tile row
-      if (MODE == kPagedTiles) {
-        const int blk = min(max(__builtin_amdgcn_readfirstlane(blk_next[0]), 0), p.num_blocks - 1);
-        row0 = static_cast<int64_t>(blk) * p.block_size + kb0 % p.block_size;
-        lim = Lk - 1 - kb0;
-      } else {
-        row0 = min(kstart + kb0, p.num_rows - 1);
-        lim = static_cast<int>(min<int64_t>(Lk - 1 - kb0, p.num_rows - 1 - row0));
-      }
-      const uint32_t limb = static_cast<uint32_t>(lim * row_stride * 2);
-      const uint16_t* kt = kbase + row0 * row_stride;
-      const uint16_t* vt = vbase + row0 * row_stride;
-#pragma unroll
-      for (int x = 0; x < NLD; ++x) {
-        const bool in = trow[x] <= lim;
-        char* dst = sbuf + (wave * WROWS + x * RPI) * ROWB;
-        load_lds16(kt, in ? koff[x] : limb + kchb[x], dst);
-        load_lds16(vt, in ? voff[x] : limb + vchb[x], dst + TBYTES);
+      const uint32_t rb = min(rowb[x], f_limb);
+      if (x2 & 1)
+        load_lds16(f_v, rb + vchb[x], dst);
+      else
+        load_lds16(f_k, rb + kchb[x], dst);
+    }
+  };
+  // After a tile's loads are issued: on to the next one.
+  auto next_tile = [&]() {
+    f_kb += kPfKeys;
+    if (f_kb > khi) {  // no further tile
+      f_limb = 0;
+      return;
+    }
+    if (MODE == kPagedTiles) {
+      f_in += kPfKeys;
+      if (f_in >= p.block_size) {
+        f_in = 0;
+        ++f_page;
+        f_blk = f_next;
+        f_next = bt[min(f_page + 1, last_page)];
       }
     }
+    fetch_rows();
+    locate_tile();
   };
 
   float m_r = -INFINITY;  // running max of raw scores (x |scale| log2 e)
@@ -336,29 +362,51 @@ __global__ __launch_bounds__(kPfThreads, 2) void paged_prefill_attn(PrefillParam
 #pragma unroll
     for (int db = 0; db < NDB; ++db) acc[db][r] = 0.f;
 
-  auto step = [&](int it, char* cur, char* nxt) {
+  const uint32_t lds0 = lds_addr(smem0), lds1 = lds_addr(smem1);
+  // One tile: scores, softmax, P.V.  The next tile's loads go out between the score
+  // MFMAs, one per k-step: issued together behind the barrier, the eight loads of all
+  // four waves queued at the address unit for ~540-660 of a step's ~2900 (one wave per
+  // SIMD) to ~3800 cycles (two), with the wave stalled at each.  4 x 4096 566 -> 530 us,
+  // two 250-512-token chunks behind 8k-24k cached keys 452 -> 383 us.  After the last
+  // tile they re-read one row of it (no branch in the MFMA sequence).
+  auto step = [&](int it, const char* cur, uint32_t nxt) {
     const int kb0 = kt0 + it * kPfKeys;
-    // Tile it has landed in LDS (own loads, then everyone's); then start the
-    // next tile into the other buffer, whose readers finished before this barrier.
+    // Tile it has landed in LDS (own loads, then everyone's); the next tile goes
+    // into the other buffer, whose readers finished before this barrier.
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();
-    if (it + 1 < ntiles) issue_tile(kb0 + kPfKeys, nxt);
-    if (wave_active && kb0 <= wave_hi && kb0 + kPfKeys - 1 >= wave_lo) {
+    {
       const uint4* sk = reinterpret_cast<const uint4*>(cur);
       const char* sv = cur + TBYTES;
 
       // S^T of two 32-key blocks: lane l holds keys 8 (r / 4) + 4 half + r % 4
-      // of block kb for its row.
+      // of block kb for its row.  Operands are read kAhead k-steps early (2, 3 and 4
+      // measured within 1 % of 1).
+      constexpr int kAhead = 1;
+      static_assert(2 * NLD == KS, "one load per k-step");
       floatx16 sc[2];
+      uint4 ka[kAhead + 1][2];
+      auto read_k = [&](int ks) {
 #pragma unroll
-      for (int kb = 0; kb < 2; ++kb) {
+        for (int kb = 0; kb < 2; ++kb)
+          ka[ks % (kAhead + 1)][kb] = sk[(kb * 32 + r32) * CH + ((2 * ks + half) ^ kswz<D>(r32))];
+      };
+#pragma unroll
+      for (int kb = 0; kb < 2; ++kb)
 #pragma unroll
         for (int r = 0; r < 16; ++r) sc[kb][r] = 0.f;
 #pragma unroll
-        for (int ks = 0; ks < KS; ++ks) {
-          const uint4 ka = sk[(kb * 32 + r32) * CH + ((2 * ks + half) ^ kswz<D>(r32))];
-          sc[kb] = mfma32x32x16(Tag{}, ka, qb[ks], sc[kb]);
-        }
+      for (int ks = 0; ks < kAhead; ++ks) read_k(ks);
+      // The score MFMAs ahead of the other workgroup's waves: 16 x 1024 186.6 -> 181.7 us,
+      // 4 x 4096 unchanged; P.V too measured 1-8 % slower.
+      __builtin_amdgcn_s_setprio(1);
+#pragma unroll
+      for (int ks = 0; ks < KS; ++ks) {
+        if (ks + kAhead < KS) read_k(ks + kAhead);
+#pragma unroll
+        for (int kb = 0; kb < 2; ++kb) sc[kb] = mfma32x32x16(Tag{}, ka[ks % (kAhead + 1)][kb], qb[ks], sc[kb]);
+        issue_load(ks, nxt);
+        __builtin_amdgcn_sched_barrier(0);
       }
 
       // Mask only where the tile crosses some row's key range.
@@ -373,11 +421,22 @@ __global__ __launch_bounds__(kPfThreads, 2) void paged_prefill_attn(PrefillParam
             sc[kb][r] = (key > hi_r || key < lo_r) ? -INFINITY : sc[kb][r];
           }
       }
-      float mt = -INFINITY;
+      __builtin_amdgcn_s_setprio(0);
+
+      // Row maximum: four independent chains of three-way maxima.
+      float mc[4];
 #pragma unroll
-      for (int kb = 0; kb < 2; ++kb)
-#pragma unroll
-        for (int r = 0; r < 16; ++r) mt = fmaxf(mt, sc[kb][r]);
+      for (int c = 0; c < 4; ++c) {
+        const floatx16& v = sc[c / 2];
+        const int r = 8 * (c % 2);
+        mc[c] = fmaxf(fmaxf(v[r], v[r + 1]), v[r + 2]);
+        mc[c] = fmaxf(fmaxf(mc[c], v[r + 3]), v[r + 4]);
+        mc[c] = fmaxf(fmaxf(mc[c], v[r + 5]), v[r + 6]);
+      }
+      float mt = fmaxf(fmaxf(mc[0], mc[1]), sc[0][7]);
+      mt = fmaxf(fmaxf(mt, mc[2]), sc[0][15]);
+      mt = fmaxf(fmaxf(mt, mc[3]), sc[1][7]);
+      mt = fmaxf(mt, sc[1][15]);
       {
         const auto sw = __builtin_amdgcn_permlane32_swap(__float_as_uint(mt), __float_as_uint(mt), false, false);
         const float a = __uint_as_float(sw[0]), b = __uint_as_float(sw[1]);
@@ -445,14 +504,14 @@ __global__ __launch_bounds__(kPfThreads, 2) void paged_prefill_attn(PrefillParam
           }
         }
     }
-    // Block-table entries for the tile after next, once this tile's LDS reads
-    // are issued (they complete under the next barrier's wait).
-    if (it + 2 < ntiles) fetch_blocks(kb0 + 2 * kPfKeys);
+    next_tile();
   };
   if (ntiles > 0) {
-    fetch_blocks(kt0);
-    issue_tile(kt0, smem0);
-    if (ntiles > 1) fetch_blocks(kt0 + kPfKeys);
+    fetch_rows();
+    locate_tile();
+#pragma unroll
+    for (int x = 0; x < 2 * NLD; ++x) issue_load(x, lds0);
+    next_tile();
   }
   // The queries load while the first tile is in flight: k-step ks takes dims
   // 16 ks + 8 half .. + 7.
@@ -466,10 +525,23 @@ __global__ __launch_bounds__(kPfThreads, 2) void paged_prefill_attn(PrefillParam
     }
   }
 
-  for (int it = 0; it < ntiles; it += 2) {
-    step(it, smem0, smem1);
-    if (it + 1 < ntiles) step(it + 1, smem1, smem0);
+  if (wave_active) {
+    for (int it = 0; it < ntiles; it += 2) {
+      step(it, smem0, lds1);
+      if (it + 1 < ntiles) step(it + 1, smem1, lds0);
+    }
+  } else {
+    // A wave without rows only loads its share of the tiles (a branch around the math
+    // inside step would cost every wave copies of its accumulators where it joins).
+    for (int it = 0; it < ntiles; ++it) {
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+      __syncthreads();
+#pragma unroll
+      for (int x = 0; x < 2 * NLD; ++x) issue_load(x, it % 2 == 0 ? lds1 : lds0);
+      next_tile();
+    }
   }
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the last step's loads, before the wave ends
 
   // out[row][d] for d = 32 db + 8 q + 4 half + e (register 4 q + e), normalised
   // by the row total (both halves of the keys).
