@@ -322,6 +322,31 @@ void paged_prefill_attention(void* out, const void* q, const void* k_cache, cons
                              float softmax_scale, int dtype, void* stream);
 
 /*
+ * paged_prefill_attention with a workspace, for queries behind a long cached context
+ * (a chunk of a prompt, a prefix hit): where the row tiles alone would leave most of
+ * the chip idle or end unevenly, their keys are split over equal workgroups, whose
+ * fp32 partial rows (in the workspace, no initialisation needed) a second kernel joins
+ * by their log-sum-exps.  No reference counterpart.  Same results within rounding;
+ * where splitting does not pay, or with a workspace that is NULL, not 16-byte aligned
+ * or smaller than prefill_attention_workspace_size(...), it is
+ * paged_prefill_attention itself.  Calls that share a workspace must not overlap in
+ * time.
+ */
+void paged_prefill_attention_workspace(void* out, const void* q, const void* k_cache, const void* v_cache,
+                                       const uint32_t* cu_seqlens_q, const uint32_t* cu_seqlens_k,
+                                       const int32_t* block_table, int64_t max_blocks_per_seq, int64_t num_blocks,
+                                       int64_t batch, int64_t num_heads, int64_t num_kv_heads, int64_t head_dim,
+                                       int64_t page_block_size, int64_t max_seqlen_q, int64_t max_seqlen_k,
+                                       int32_t window_left, float softmax_scale, void* workspace,
+                                       size_t workspace_bytes, int dtype, void* stream);
+
+/* Bytes of workspace (at most 68 MB with 256 CUs at head_dim 128) with which
+ * paged_prefill_attention_workspace and varlen_prefill_attention_workspace split these
+ * arguments' keys; 0 where they run as the plain entries. */
+size_t prefill_attention_workspace_size(int64_t batch, int64_t num_heads, int64_t num_kv_heads, int64_t head_dim,
+                                        int64_t max_seqlen_q, int64_t max_seqlen_k, int32_t window_left);
+
+/*
  * The same attention over contiguous K/V.  Replaces
  * candle_flash_attn::flash_attn_varlen(q, k, v, cu_seqlens_q, cu_seqlens_k,
  * max_seqlen_q, max_seqlen_k, softmax_scale, causal = true) of prefill_attn,
@@ -336,6 +361,14 @@ void varlen_prefill_attention(void* out, const void* q, const void* k, const voi
                               int64_t num_kv_heads, int64_t head_dim, int64_t max_seqlen_q,
                               int64_t max_seqlen_k, int32_t window_left, float softmax_scale,
                               int dtype, void* stream);
+
+/* varlen_prefill_attention with a workspace, as paged_prefill_attention_workspace. */
+void varlen_prefill_attention_workspace(void* out, const void* q, const void* k, const void* v,
+                                        const uint32_t* cu_seqlens_q, const uint32_t* cu_seqlens_k,
+                                        int64_t total_k, int64_t batch, int64_t num_heads,
+                                        int64_t num_kv_heads, int64_t head_dim, int64_t max_seqlen_q,
+                                        int64_t max_seqlen_k, int32_t window_left, float softmax_scale,
+                                        void* workspace, size_t workspace_bytes, int dtype, void* stream);
 
 /*
  * The attention prologue fused with the KV append.  Replaces, per token t, the

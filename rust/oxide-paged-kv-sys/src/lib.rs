@@ -300,6 +300,44 @@ extern "C" {
         stream: HipStream,
     );
 
+    /// paged_prefill_attention with a workspace: queries behind a long cached context have their
+    /// keys split over equal workgroups and the partial rows joined (the plain call elsewhere).
+    pub fn paged_prefill_attention_workspace(
+        out: *mut c_void,
+        q: *const c_void,
+        k_cache: *const c_void,
+        v_cache: *const c_void,
+        cu_seqlens_q: *const u32,
+        cu_seqlens_k: *const u32,
+        block_table: *const i32,
+        max_blocks_per_seq: i64,
+        num_blocks: i64,
+        batch: i64,
+        num_heads: i64,
+        num_kv_heads: i64,
+        head_dim: i64,
+        page_block_size: i64,
+        max_seqlen_q: i64,
+        max_seqlen_k: i64,
+        window_left: i32,
+        softmax_scale: f32,
+        workspace: *mut c_void,
+        workspace_bytes: usize,
+        dtype: c_int,
+        stream: HipStream,
+    );
+
+    /// Bytes of workspace with which the workspace forms split; 0 where they do not.
+    pub fn prefill_attention_workspace_size(
+        batch: i64,
+        num_heads: i64,
+        num_kv_heads: i64,
+        head_dim: i64,
+        max_seqlen_q: i64,
+        max_seqlen_k: i64,
+        window_left: i32,
+    ) -> usize;
+
     /// flash_attn_varlen(.., causal = true) over contiguous K/V (prefill_attn, flash_attn.rs:15-37).
     pub fn varlen_prefill_attention(
         out: *mut c_void,
@@ -317,6 +355,29 @@ extern "C" {
         max_seqlen_k: i64,
         window_left: i32,
         softmax_scale: f32,
+        dtype: c_int,
+        stream: HipStream,
+    );
+
+    /// varlen_prefill_attention with a workspace, as paged_prefill_attention_workspace.
+    pub fn varlen_prefill_attention_workspace(
+        out: *mut c_void,
+        q: *const c_void,
+        k: *const c_void,
+        v: *const c_void,
+        cu_seqlens_q: *const u32,
+        cu_seqlens_k: *const u32,
+        total_k: i64,
+        batch: i64,
+        num_heads: i64,
+        num_kv_heads: i64,
+        head_dim: i64,
+        max_seqlen_q: i64,
+        max_seqlen_k: i64,
+        window_left: i32,
+        softmax_scale: f32,
+        workspace: *mut c_void,
+        workspace_bytes: usize,
         dtype: c_int,
         stream: HipStream,
     );

@@ -136,6 +136,33 @@ def test_prefill_random_shapes_vs_oracle(device, case):
     assert_attn_close(got, oracle.prefill_attention(q, kc, vc, cuq, cuk, scale, table, window, dtype))
 
 
+# Queries behind long cached contexts, whose keys are split over workgroups: the piece
+# and tile edges, sequences with nothing to split or no queries, the smallest batch and
+# the largest that is split (64), rows of 128 that groups of 7 and 5 do not fill.
+BALANCED = [
+    # (lq, lk, Hq, Hkv, D, BS, window, dtype)
+    ([1], [1500], 32, 8, 128, 256, -1, "bf16"),                       # one row tile, pieces of 8 steps
+    ([33, 1], [1025, 1600], 32, 8, 128, 64, -1, "f16"),               # one row past a row tile
+    ([40, 0, 70, 12], [2100, 900, 1000, 12], 28, 4, 128, 256, -1, "bf16"),  # G=7; no queries; no cached keys
+    ([30, 18], [1400, 5], 40, 8, 64, 16, -1, "bf16"),                 # Lk < Lq beside a split one; per-row pages
+    ([64, 64], [3000, 1900], 16, 8, 128, 256, 1000, "f16"),           # window over several pieces
+    ([1] * 63 + [9], [600 + 31 * i for i in range(64)], 16, 2, 64, 32, -1, "bf16"),  # 64 sequences
+]
+
+
+@pytest.mark.parametrize("case", BALANCED, ids=[f"b{i}" for i in range(len(BALANCED))])
+def test_prefill_behind_long_context_vs_oracle(device, case):
+    from oxide_paged_kv import _lib
+
+    lq, lk, Hq, Hkv, D, BS, window, dtype = case
+    assert _lib.load().prefill_attention_workspace_size(len(lq), Hq, Hkv, D, max(lq), max(lk), window) > 0
+    q, kc, vc, cuq, cuk, table = _case(51, lq, lk, Hq, Hkv, D, BS, dtype)
+    scale = 1.0 / math.sqrt(D)
+    print(f"prefill balanced lq={lq[:4]} lk={lk[:4]} Hq={Hq} Hkv={Hkv} D={D} BS={BS} w={window} {dtype}", flush=True)
+    got = to_f32(_gpu(device, q, kc, vc, cuq, cuk, table, scale, window, dtype))
+    assert_attn_close(got, oracle.prefill_attention(q, kc, vc, cuq, cuk, scale, table, window, dtype))
+
+
 @pytest.mark.parametrize("case", [CASES[1], CASES[4], CASES[7]], ids=["prefix", "window", "d64"])
 def test_prefill_contiguous_equals_paged(device, case):
     """flash_attn_varlen form (contiguous K/V): same kernel, so bit-identical to the paged

@@ -94,10 +94,103 @@ struct PrefillParams {
   int dec_batch;
   int* shared_out;  // the number of shared blocks found (written by workgroup 0)
   int pair;         // 1: each workgroup takes row tiles n - 1 - i and then i of its unit
+  // Balanced launch (kernel instances with kSplit): the most pieces it cuts, and the
+  // batch size.  Partial rows go to part_o / part_lse, row piece * kPfRows + row.
+  int max_pieces;
+  int slots;       // workgroups that run at once
+  int batch;
+  int* piece_len;  // the piece length chosen (workgroup 0 writes it, the merge reads it)
 };
 
 __device__ __forceinline__ int clamp_len(int64_t n, int cap) {
   return static_cast<int>(n < 0 ? 0 : (n > cap ? cap : n));
+}
+
+// Balanced launch: the 64-key steps of every row tile of sequence b are cut into n_b
+// equal pieces, one workgroup each.  Pieces are numbered sequence by sequence, inside
+// one by kv head, then key range, then row tile: neighbouring workgroups, on one XCD,
+// walk the same keys for different rows, so K/V comes from that XCD's L2.  (Ranges of
+// equal length over the rows' steps laid end to end balance perfectly, but every
+// workgroup then streams its own keys: 337 us for two chunks behind 16k-24k keys
+// against 300-310 with the pieces.)  The piece length is the shortest for which all
+// pieces run at once (slots workgroups), or in two rounds where rounding to whole
+// pieces costs the single round more than an eighth.
+// Lane b of every wave holds sequence b's entry (so at most 64 sequences).
+constexpr int kPfSplitBatch = 64;
+constexpr int kPfMinPiece = 8;
+struct SeqPieces {
+  int q;       // clamped query count
+  int tiles;   // row tiles per kv head
+  int steps;   // steps of a tile (of its last tile; earlier ones leave a few empty)
+  int n;       // pieces of a tile
+  int first;   // number of its first piece
+  int total;   // all sequences' pieces (the same in every lane)
+};
+__host__ __device__ __forceinline__ int steps_per_tile(int keys, int window_left, int tokens_per_wg) {
+  const int all = (keys + kPfKeys - 1) / kPfKeys;
+  if (window_left < 0 || window_left >= keys) return all;
+  const int n = (window_left + tokens_per_wg + 2 * kPfKeys - 2) / kPfKeys;
+  return n < all ? n : all;
+}
+// Inclusive sums over the lanes (lane 63 holds the total), on the VALU.
+__device__ __forceinline__ int wave_scan(int v) {
+  v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, false);  // row_shr:1
+  v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, false);  // row_shr:2
+  v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, false);  // row_shr:4
+  v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, false);  // row_shr:8
+  v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, false);  // row_bcast:15, rows 1 and 3
+  v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false);  // row_bcast:31, rows 2 and 3
+  return v;
+}
+__device__ __forceinline__ int wave_total(int v) { return __builtin_amdgcn_readlane(wave_scan(v), 63); }
+
+// The shortest piece length, at least kPfMinPiece, at which the sequences (units row
+// tiles of steps steps each, per lane) make at most `slots` pieces.
+__device__ __forceinline__ int shortest_piece(int units, int steps, int slots) {
+  // units * steps / len <= pieces <= units * (steps / len + 1) bound the bisection.
+  const int tiles = wave_total(units);
+  const int work = wave_total(units * steps);
+  int lo = max(kPfMinPiece, (work + slots - 1) / slots);
+  int hi = slots > tiles ? max(lo, (work + slots - tiles - 1) / (slots - tiles)) : INT32_MAX / 2;
+  while (lo < hi) {
+    const int mid = (lo + hi) / 2;
+    if (wave_total(units * ((steps + mid - 1) / mid)) <= slots)
+      hi = mid;
+    else
+      lo = mid + 1;
+  }
+  return lo;
+}
+// kMerge: the piece length comes from the first pass.
+template <bool kMerge>
+__device__ __forceinline__ SeqPieces seq_pieces(const PrefillParams& p) {
+  const int lane = threadIdx.x & 63;
+  SeqPieces s{};
+  int k = 0;
+  if (lane < p.batch) {
+    s.q = clamp_len(static_cast<int64_t>(p.cu_seqlens_q[lane + 1]) - p.cu_seqlens_q[lane], p.max_seqlen_q);
+    k = clamp_len(static_cast<int64_t>(p.cu_seqlens_k[lane + 1]) - p.cu_seqlens_k[lane], p.max_seqlen_k);
+  }
+  s.tiles = (s.q + p.tokens_per_wg - 1) / p.tokens_per_wg;
+  s.steps = max(steps_per_tile(k, p.window_left, p.tokens_per_wg), 1);
+  const int units = p.num_kv_heads * s.tiles;  // row tiles of the sequence
+  int len;
+  if (kMerge) {
+    len = __builtin_amdgcn_readfirstlane(*p.piece_len);
+  } else {
+    len = shortest_piece(units, s.steps, p.max_pieces);
+    if (p.max_pieces > p.slots && wave_total(units) <= p.slots) {
+      const int one = shortest_piece(units, s.steps, p.slots);
+      if (8 * one <= 18 * len) len = one;
+    }
+    if (blockIdx.x == 0 && threadIdx.x == 0) *p.piece_len = len;
+  }
+  s.n = (s.steps + len - 1) / len;
+  const int mine = units * s.n;
+  const int sum = wave_scan(mine);
+  s.first = sum - mine;
+  s.total = __builtin_amdgcn_readlane(sum, 63);
+  return s;
 }
 
 // LDS tile layouts (64 keys, row = one key's head slice of 2*D bytes):
@@ -150,7 +243,7 @@ enum PrefillAddressing {
   kPagedRows = 2,   // paged, any block_size: a block lookup per row
 };
 
-template <class Tag, int D, int MODE, bool kPrefix, bool kPair = false>
+template <class Tag, int D, int MODE, bool kPrefix, bool kPair = false, bool kSplit = false>
 __global__ __launch_bounds__(kPfThreads, 2) void paged_prefill_attn(PrefillParams p) {
   constexpr int CH = D / 8;                  // 16-byte chunks per head row
   constexpr int KS = D / 16;                 // MFMA k-steps of Q.K (16 dims each)
@@ -171,21 +264,45 @@ __global__ __launch_bounds__(kPfThreads, 2) void paged_prefill_attn(PrefillParam
   // XCD-aware work item: unit (sequence, kv head) u sits on XCD u % 8 and its
   // tiles are consecutive workgroups there, heaviest first.  Shared-prefix pass:
   // unit (key split, kv head), all of them over table row 0 (the shared entries).
+  // Balanced launch: XCD x takes the x-th eighth of the pieces.
   const int i = blockIdx.x;
   const int j = i / kPfXcds;
   const int wpu = kPair ? (p.tiles_per_unit + 1) / 2 : p.tiles_per_unit;  // workgroups per unit
   const int u = (j / wpu) * kPfXcds + i % kPfXcds;
-  if (u >= p.units) return;
+  if (!kSplit && u >= p.units) return;
   const int jj = j % wpu;
   for (int pass = 0; pass < (kPair ? 2 : 1); ++pass) {
-  const int tile = pass == 0 ? p.tiles_per_unit - 1 - jj : jj;
-  if (pass == 1) {
-    if (tile >= p.tiles_per_unit - 1 - jj) break;  // the middle tile of an odd count: done
-    __syncthreads();  // the previous tile's last LDS reads before this tile's first loads
+  int tile, b, kh, split = 0;
+  int piece = 0, s0 = 0, s1 = 0;  // kSplit: the piece and its steps of the tile
+  bool whole = true;
+  if constexpr (kSplit) {
+    const SeqPieces seqs = seq_pieces<false>(p);
+    const int per_xcd = (seqs.total + kPfXcds - 1) / kPfXcds;
+    piece = (i % kPfXcds) * per_xcd + j;
+    if (j >= per_xcd || piece >= min(seqs.total, p.max_pieces)) return;
+    // The last sequence whose first piece is not past this one (sequences without
+    // queries share their successor's first, so it is the one that holds it).
+    b = 63 - __builtin_clzll(__ballot(static_cast<int>(threadIdx.x & 63) < p.batch && seqs.first <= piece));
+    const int in_seq = piece - __builtin_amdgcn_readlane(seqs.first, b);
+    const int tiles = __builtin_amdgcn_readlane(seqs.tiles, b);
+    const int steps = __builtin_amdgcn_readlane(seqs.steps, b);
+    const int n = __builtin_amdgcn_readlane(seqs.n, b);
+    kh = in_seq / (tiles * n);
+    const int x = in_seq / tiles % n;
+    tile = in_seq % tiles;
+    s0 = static_cast<int>(static_cast<int64_t>(steps) * x / n);
+    s1 = static_cast<int>(static_cast<int64_t>(steps) * (x + 1) / n);
+    whole = n == 1;
+  } else {
+    tile = pass == 0 ? p.tiles_per_unit - 1 - jj : jj;
+    if (pass == 1) {
+      if (tile >= p.tiles_per_unit - 1 - jj) break;  // the middle tile of an odd count: done
+      __syncthreads();  // the previous tile's last LDS reads before this tile's first loads
+    }
+    b = kPrefix ? 0 : u / p.num_kv_heads;
+    kh = u % p.num_kv_heads;
+    split = kPrefix ? u / p.num_kv_heads : 0;
   }
-  const int b = kPrefix ? 0 : u / p.num_kv_heads;
-  const int kh = u % p.num_kv_heads;
-  const int split = kPrefix ? u / p.num_kv_heads : 0;
 
   int Lq, Lk;
   if constexpr (kPrefix) {
@@ -208,10 +325,16 @@ __global__ __launch_bounds__(kPfThreads, 2) void paged_prefill_attn(PrefillParam
 
   // Key range of the workgroup: [klo, khi] (empty when khi < klo).  Shared-prefix
   // pass: the split's keys, every row seeing all of them but those before its window.
-  const int khi = kPrefix ? min(Lk, (split + 1) * p.split_keys) - 1 : min(Lk - 1, t1 - 1 + off);
+  // Balanced launch: steps s0 .. s1 - 1 of the tile's keys.
+  int khi = kPrefix ? min(Lk, (split + 1) * p.split_keys) - 1 : min(Lk - 1, t1 - 1 + off);
   const int klo = kPrefix ? split * p.split_keys : (W >= 0 ? max(0, t0 + off - W) : 0);
-  const int kt0 = klo & ~(kPfKeys - 1);
-  const int ntiles = khi >= klo ? (khi - kt0) / kPfKeys + 1 : 0;
+  int kt0 = klo & ~(kPfKeys - 1);
+  if constexpr (kSplit) {
+    khi = min(khi, kt0 + s1 * kPfKeys - 1);
+    kt0 += s0 * kPfKeys;
+    if (khi < kt0) khi = -1;  // past the tile's last key
+  }
+  const int ntiles = khi >= klo && khi >= kt0 ? (khi - kt0) / kPfKeys + 1 : 0;
 
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int lane = threadIdx.x & 63;
@@ -546,12 +669,14 @@ __global__ __launch_bounds__(kPfThreads, 2) void paged_prefill_attn(PrefillParam
   // out[row][d] for d = 32 db + 8 q + 4 half + e (register 4 q + e), normalised
   // by the row total (both halves of the keys).
   lsum = sum_over_halves(lsum);
-  if (kPrefix && valid) {
+  const bool partial = kPrefix || !whole;
+  if (partial && valid) {
     // Normalised partial row and its log2-sum-exp (scores are in units of
     // |scale| log2 e, as the decode passes' partials).
     const float l = lsum;
     const float inv = l > 0.f ? 1.f / l : 0.f;
-    const int64_t prow = p.pre_row0 + static_cast<int64_t>(split) * p.dec_batch * p.num_heads + qrow;
+    const int64_t prow = kSplit ? static_cast<int64_t>(piece) * kPfRows + rr
+                                : p.pre_row0 + static_cast<int64_t>(split) * p.dec_batch * p.num_heads + qrow;
     float* po = p.part_o + prow * D + 4 * half;
 #pragma unroll
     for (int db = 0; db < NDB; ++db)
@@ -578,7 +703,110 @@ __global__ __launch_bounds__(kPfThreads, 2) void paged_prefill_attn(PrefillParam
   }
 }
 
+// Joins the pieces of the row tiles that the balanced launch cut, weighted by their
+// log-sum-exps: a workgroup of 256 threads per 16 rows of a (sequence, kv head, row
+// tile), D / 4 threads per row.  Bound by its reads (512 B per piece and row at D =
+// 128); four pieces' rows are in flight per thread.
+constexpr int kPfMergeRows = 16;
+template <class Tag, int D>
+__global__ __launch_bounds__(256) void paged_prefill_merge(PrefillParams p) {
+  constexpr int TPR = D / 4;             // threads per row
+  constexpr int RPP = 256 / TPR;         // rows per pass
+  constexpr int PARTS = kPfRows / kPfMergeRows;
+  const SeqPieces seqs = seq_pieces<true>(p);
+  const int part = blockIdx.x % PARTS;
+  const int x = blockIdx.x / PARTS;
+  const int b = x / (p.num_kv_heads * p.tiles_per_unit);
+  const int kh = x / p.tiles_per_unit % p.num_kv_heads;
+  const int tile = x % p.tiles_per_unit;
+  const int tiles = __builtin_amdgcn_readlane(seqs.tiles, b);
+  const int n = __builtin_amdgcn_readlane(seqs.n, b);
+  if (tile >= tiles || n == 1) return;
+  const int first = __builtin_amdgcn_readlane(seqs.first, b) + kh * n * tiles + tile;
+  const int Lq = __builtin_amdgcn_readlane(seqs.q, b);
+  const int64_t q0 = p.cu_seqlens_q[b];
+  const int G = p.group;
+  const int c = threadIdx.x % TPR;
+  const int r1 = (part + 1) * kPfMergeRows;
+  for (int r = part * kPfMergeRows + threadIdx.x / TPR; r < r1; r += RPP) {
+    const int tq = tile * p.tokens_per_wg + r / G;
+    if (r >= p.tokens_per_wg * G || tq >= Lq) break;
+    auto row = [&](int y) { return static_cast<int64_t>(first + min(y, n - 1) * tiles) * kPfRows + r; };
+    float m = -INFINITY, l = 0.f;
+    float4 o = make_float4(0.f, 0.f, 0.f, 0.f);
+    for (int y = 0; y < n; y += 4) {
+      float e[4];
+      float4 v[4];
+#pragma unroll
+      for (int z = 0; z < 4; ++z) e[z] = y + z < n ? p.part_lse[row(y + z)] : -INFINITY;
+#pragma unroll
+      for (int z = 0; z < 4; ++z) v[z] = *reinterpret_cast<const float4*>(p.part_o + row(y + z) * D + 4 * c);
+      const float mn = fmaxf(fmaxf(m, fmaxf(e[0], e[1])), fmaxf(e[2], e[3]));
+      if (mn == -INFINITY) continue;
+      const float a = __builtin_amdgcn_exp2f(m - mn);
+      m = mn;
+      l *= a;
+      o.x *= a;
+      o.y *= a;
+      o.z *= a;
+      o.w *= a;
+#pragma unroll
+      for (int z = 0; z < 4; ++z) {
+        const float f = __builtin_amdgcn_exp2f(e[z] - mn);
+        l += f;
+        o.x += f * v[z].x;
+        o.y += f * v[z].y;
+        o.z += f * v[z].z;
+        o.w += f * v[z].w;
+      }
+    }
+    const float inv = l > 0.f ? 1.f / l : 0.f;
+    uint2 out;
+    out.x = pack2(Tag{}, o.x * inv, o.y * inv);
+    out.y = pack2(Tag{}, o.z * inv, o.w * inv);
+    *reinterpret_cast<uint2*>(static_cast<uint16_t*>(p.out) + ((q0 + tq) * p.num_heads + kh * G + r % G) * D + 4 * c) =
+        out;
+  }
+}
+
 int64_t ceil_div64(int64_t a, int64_t b) { return (a + b - 1) / b; }
+
+// The most pieces of the balanced launch, 0 = the plain grid.
+// Long cached contexts only (causal rows of a whole prompt carry unequal keys).  A step
+// (128 rows x 64 keys, D = 128) takes about 1.03 us with one workgroup on a CU and 1.9
+// us with two; the pieces' fp32 rows and the merge add ~15 % and ~6 us.  Taken where
+// that beats the plain grid; a batch is expected to be ragged, so that it has ~15 %
+// less work than its longest sequence says.  Measured, plain -> balanced: two chunks of
+// 342-512 tokens behind 16k-24k keys 390 -> 310 us, 512 behind 8k 162 -> 87, 64 behind
+// 32k 586 -> 61, 16 x 16 behind 4k-8k 156 -> 92; left alone: 1024 behind 2k (64 vs 67
+// split), 2048 behind 8k (297 vs 316).
+int balanced_pieces(int64_t batch, int64_t num_heads, int64_t num_kv_heads, int64_t head_dim, int64_t max_seqlen_q,
+                    int64_t max_seqlen_k, int64_t window_left) {
+  if (batch <= 0 || batch > kPfSplitBatch || max_seqlen_q <= 0 || num_kv_heads <= 0 || num_heads < num_kv_heads ||
+      num_heads / num_kv_heads > kPfRows || max_seqlen_k < 2 * max_seqlen_q || max_seqlen_k > INT32_MAX / 2)
+    return 0;
+  const int64_t cus = oxide::device_cu_count();
+  const int64_t slots = 2 * cus;
+  const int64_t tpw = kPfRows / (num_heads / num_kv_heads);
+  const int64_t tiles = batch * num_kv_heads * ceil_div64(max_seqlen_q, tpw);
+  if (tiles > 2 * slots) return 0;
+  const int64_t w = window_left < 0 || window_left >= max_seqlen_k ? -1 : window_left;
+  const int64_t steps = steps_per_tile(static_cast<int>(max_seqlen_k), static_cast<int>(w), static_cast<int>(tpw));
+  const int64_t pieces = std::min(2 * slots, tiles * ceil_div64(steps, kPfMinPiece));
+  if (pieces <= tiles || tiles * steps > INT32_MAX / 2) return 0;  // the kernel sums steps in 32 bits
+  const double unit = head_dim / 128.0;
+  const double plain = unit * ceil_div64(tiles, slots) * steps * (tiles > cus ? 1.9 : 1.03);
+  const double split =
+      std::max(unit * tiles * steps / slots * 1.9 * 1.15, unit * kPfMinPiece * 1.03) * (batch > 1 ? 0.85 : 1.0) + 6.0;
+  return split < plain ? static_cast<int>(pieces) : 0;
+}
+size_t balanced_rows_bytes(int pieces, int64_t head_dim) {
+  return static_cast<size_t>(pieces) * kPfRows * static_cast<size_t>(head_dim) * sizeof(float);
+}
+// Partial rows, their log-sum-exps, the piece length.
+size_t balanced_bytes(int pieces, int64_t head_dim) {
+  return balanced_rows_bytes(pieces, head_dim) + (static_cast<size_t>(pieces) * kPfRows + 1) * sizeof(float);
+}
 
 template <class Tag, int D>
 void launch_mode(const PrefillParams& p, dim3 grid, hipStream_t s) {
@@ -600,6 +828,20 @@ void launch_mode(const PrefillParams& p, dim3 grid, hipStream_t s) {
 }
 
 template <class Tag, int D>
+void launch_balanced(const PrefillParams& p, hipStream_t s) {
+  const dim3 grid(static_cast<unsigned>(ceil_div64(p.max_pieces, kPfXcds) * kPfXcds));
+  if (p.block_table == nullptr)
+    hipLaunchKernelGGL((paged_prefill_attn<Tag, D, kContiguous, false, false, true>), grid, dim3(kPfThreads), 0, s, p);
+  else if (p.block_size % kPfKeys == 0)
+    hipLaunchKernelGGL((paged_prefill_attn<Tag, D, kPagedTiles, false, false, true>), grid, dim3(kPfThreads), 0, s, p);
+  else
+    hipLaunchKernelGGL((paged_prefill_attn<Tag, D, kPagedRows, false, false, true>), grid, dim3(kPfThreads), 0, s, p);
+  oxide::check_launch();
+  hipLaunchKernelGGL((paged_prefill_merge<Tag, D>), dim3(static_cast<unsigned>(
+                     kPfRows / kPfMergeRows * p.units * p.tiles_per_unit)), dim3(256), 0, s, p);
+}
+
+template <class Tag, int D>
 void launch_prefix_mode(const PrefillParams& p, dim3 grid, hipStream_t s) {
   if (p.block_size % kPfKeys == 0)
     hipLaunchKernelGGL((paged_prefill_attn<Tag, D, kPagedTiles, true>), grid, dim3(kPfThreads), 0, s, p);
@@ -609,6 +851,10 @@ void launch_prefix_mode(const PrefillParams& p, dim3 grid, hipStream_t s) {
 
 template <class Tag>
 bool launch_prefill(const PrefillParams& p, int head_dim, hipStream_t s) {
+  if (p.max_pieces > 0) {
+    head_dim == 128 ? launch_balanced<Tag, 128>(p, s) : launch_balanced<Tag, 64>(p, s);
+    return true;
+  }
   const int64_t units8 = ceil_div64(p.units, kPfXcds) * kPfXcds;
   const dim3 grid(static_cast<unsigned>(units8 * (p.pair ? (p.tiles_per_unit + 1) / 2 : p.tiles_per_unit)));
   if (head_dim == 128) {
@@ -627,7 +873,7 @@ void prefill_impl(void* out, const void* q, const void* k, const void* v, const 
                   int64_t num_blocks, int64_t num_rows, int64_t batch, int64_t num_heads,
                   int64_t num_kv_heads, int64_t head_dim, int64_t page_block_size,
                   int64_t max_seqlen_q, int64_t max_seqlen_k, int32_t window_left,
-                  float softmax_scale, int dtype, void* stream) {
+                  float softmax_scale, void* workspace, size_t workspace_bytes, int dtype, void* stream) {
   if (dtype != OXIDE_DTYPE_BF16 && dtype != OXIDE_DTYPE_F16) {
     oxide::set_error(OXIDE_ERR_UNSUPPORTED_DTYPE);
     return;
@@ -699,6 +945,17 @@ void prefill_impl(void* out, const void* q, const void* k, const void* v, const 
   p.block_size = static_cast<int>(block_table ? page_block_size : 1);
   p.window_left = window_left < 0 ? -1 : window_left;
   p.scale_log2 = softmax_scale * 1.4426950408889634f;
+  p.batch = static_cast<int>(batch);
+  if (workspace != nullptr && oxide::aligned16(workspace)) {
+    const int pieces = balanced_pieces(batch, num_heads, num_kv_heads, head_dim, max_seqlen_q, max_seqlen_k, window_left);
+    if (pieces > 0 && workspace_bytes >= balanced_bytes(pieces, head_dim)) {
+      p.max_pieces = pieces;
+      p.slots = 2 * oxide::device_cu_count();
+      p.part_o = static_cast<float*>(workspace);
+      p.part_lse = reinterpret_cast<float*>(static_cast<char*>(workspace) + balanced_rows_bytes(pieces, head_dim));
+      p.piece_len = reinterpret_cast<int*>(p.part_lse + static_cast<int64_t>(pieces) * kPfRows);
+    }
+  }
   hipStream_t s = oxide::as_stream(stream);
   const bool ok = dtype == OXIDE_DTYPE_BF16 ? launch_prefill<Bf16Tag>(p, static_cast<int>(head_dim), s)
                                             : launch_prefill<F16Tag>(p, static_cast<int>(head_dim), s);
@@ -725,7 +982,30 @@ extern "C" void paged_prefill_attention(void* out, const void* q, const void* k_
   }
   prefill_impl(out, q, k_cache, v_cache, cu_seqlens_q, cu_seqlens_k, block_table, max_blocks_per_seq,
                num_blocks, 0, batch, num_heads, num_kv_heads, head_dim, page_block_size, max_seqlen_q,
-               max_seqlen_k, window_left, softmax_scale, dtype, stream);
+               max_seqlen_k, window_left, softmax_scale, nullptr, 0, dtype, stream);
+}
+
+extern "C" size_t prefill_attention_workspace_size(int64_t batch, int64_t num_heads, int64_t num_kv_heads,
+                                                         int64_t head_dim, int64_t max_seqlen_q, int64_t max_seqlen_k,
+                                                         int32_t window_left) {
+  if (head_dim != 64 && head_dim != 128) return 0;
+  const int pieces = balanced_pieces(batch, num_heads, num_kv_heads, head_dim, max_seqlen_q, max_seqlen_k, window_left);
+  return pieces > 0 ? balanced_bytes(pieces, head_dim) : 0;
+}
+
+extern "C" void paged_prefill_attention_workspace(
+    void* out, const void* q, const void* k_cache, const void* v_cache, const uint32_t* cu_seqlens_q,
+    const uint32_t* cu_seqlens_k, const int32_t* block_table, int64_t max_blocks_per_seq, int64_t num_blocks,
+    int64_t batch, int64_t num_heads, int64_t num_kv_heads, int64_t head_dim, int64_t page_block_size,
+    int64_t max_seqlen_q, int64_t max_seqlen_k, int32_t window_left, float softmax_scale, void* workspace,
+    size_t workspace_bytes, int dtype, void* stream) {
+  if (block_table == nullptr && max_seqlen_k > 0) {
+    oxide::set_error(OXIDE_ERR_INVALID_ARGUMENT);
+    return;
+  }
+  prefill_impl(out, q, k_cache, v_cache, cu_seqlens_q, cu_seqlens_k, block_table, max_blocks_per_seq,
+               num_blocks, 0, batch, num_heads, num_kv_heads, head_dim, page_block_size, max_seqlen_q,
+               max_seqlen_k, window_left, softmax_scale, workspace, workspace_bytes, dtype, stream);
 }
 
 extern "C" void varlen_prefill_attention(void* out, const void* q, const void* k, const void* v,
@@ -736,7 +1016,17 @@ extern "C" void varlen_prefill_attention(void* out, const void* q, const void* k
                                          int dtype, void* stream) {
   prefill_impl(out, q, k, v, cu_seqlens_q, cu_seqlens_k, nullptr, 0, 0, total_k, batch, num_heads,
                num_kv_heads, head_dim, 1, max_seqlen_q, max_seqlen_k, window_left, softmax_scale,
-               dtype, stream);
+               nullptr, 0, dtype, stream);
+}
+
+extern "C" void varlen_prefill_attention_workspace(
+    void* out, const void* q, const void* k, const void* v, const uint32_t* cu_seqlens_q,
+    const uint32_t* cu_seqlens_k, int64_t total_k, int64_t batch, int64_t num_heads, int64_t num_kv_heads,
+    int64_t head_dim, int64_t max_seqlen_q, int64_t max_seqlen_k, int32_t window_left, float softmax_scale,
+    void* workspace, size_t workspace_bytes, int dtype, void* stream) {
+  prefill_impl(out, q, k, v, cu_seqlens_q, cu_seqlens_k, nullptr, 0, 0, total_k, batch, num_heads,
+               num_kv_heads, head_dim, 1, max_seqlen_q, max_seqlen_k, window_left, softmax_scale,
+               workspace, workspace_bytes, dtype, stream);
 }
 
 namespace oxide {

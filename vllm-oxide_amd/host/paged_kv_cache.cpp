@@ -212,6 +212,7 @@ PrefillStep::PrefillStep(const PagedKVCache& cache, std::size_t num_heads)
 
 PrefillStep::~PrefillStep() {
   if (d_buf_) (void)hipFree(d_buf_);
+  if (d_ws_) (void)hipFree(d_ws_);
 }
 
 void PrefillStep::upload(const AttnMetadata& meta, const std::vector<std::vector<int32_t>>& block_table,
@@ -245,6 +246,18 @@ void PrefillStep::upload(const AttnMetadata& meta, const std::vector<std::vector
     check(hipMalloc(&d_buf_, total), "hipMalloc(PrefillStep)");
     cap_ = total;
   }
+  // The unwindowed size covers every window.
+  const std::size_t ws = prefill_attention_workspace_size(
+      static_cast<int64_t>(batch_), static_cast<int64_t>(num_heads_), static_cast<int64_t>(cache_.num_kv_heads()),
+      static_cast<int64_t>(cache_.head_dim()), static_cast<int64_t>(max_seqlen_q_),
+      static_cast<int64_t>(max_seqlen_k_), -1);
+  if (ws > cap_ws_) {
+    if (d_ws_) check(hipFree(d_ws_), "hipFree");
+    d_ws_ = nullptr;
+    cap_ws_ = 0;
+    check(hipMalloc(&d_ws_, ws), "hipMalloc(PrefillStep)");
+    cap_ws_ = ws;
+  }
   char* d = static_cast<char*>(d_buf_);
   check(hipMemcpyAsync(d, h_cuq_.data(), h_cuq_.size() * 4, hipMemcpyHostToDevice, stream), "upload cu_seqlens_q");
   check(hipMemcpyAsync(d + off_cuk_, h_cuk_.data(), h_cuk_.size() * 4, hipMemcpyHostToDevice, stream),
@@ -271,14 +284,13 @@ void PrefillStep::run_layer(std::size_t layer, const void* qkv, const void* q_no
                            cache_.v_cache(layer), reinterpret_cast<const int64_t*>(d + off_slots_),
                            static_cast<int64_t>(num_tokens_), Hq, Hkv, D, cache_.dtype(), stream);
   check_lib("qk_norm_rope_and_cache");
-  ::paged_prefill_attention(out, q_scratch, cache_.k_cache(layer), cache_.v_cache(layer),
-                            reinterpret_cast<const uint32_t*>(d), reinterpret_cast<const uint32_t*>(d + off_cuk_),
-                            reinterpret_cast<const int32_t*>(d + off_table_), static_cast<int64_t>(max_blocks_),
-                            static_cast<int64_t>(cache_.num_blocks()), static_cast<int64_t>(batch_), Hq, Hkv, D,
-                            static_cast<int64_t>(cache_.block_size()), static_cast<int64_t>(max_seqlen_q_),
-                            static_cast<int64_t>(max_seqlen_k_), window_left, softmax_scale, cache_.dtype(),
-                            stream);
-  check_lib("paged_prefill_attention");
+  ::paged_prefill_attention_workspace(
+      out, q_scratch, cache_.k_cache(layer), cache_.v_cache(layer), reinterpret_cast<const uint32_t*>(d),
+      reinterpret_cast<const uint32_t*>(d + off_cuk_), reinterpret_cast<const int32_t*>(d + off_table_),
+      static_cast<int64_t>(max_blocks_), static_cast<int64_t>(cache_.num_blocks()), static_cast<int64_t>(batch_), Hq,
+      Hkv, D, static_cast<int64_t>(cache_.block_size()), static_cast<int64_t>(max_seqlen_q_),
+      static_cast<int64_t>(max_seqlen_k_), window_left, softmax_scale, d_ws_, cap_ws_, cache_.dtype(), stream);
+  check_lib("paged_prefill_attention_workspace");
 }
 
 }  // namespace oxide::host

@@ -143,6 +143,8 @@ class PrefillStep {
   std::vector<int64_t> h_slots_;
   void* d_buf_ = nullptr;  // cu_q | cu_k | table | positions | slots, 256-byte aligned parts
   std::size_t cap_ = 0;
+  void* d_ws_ = nullptr;  // partial rows of calls behind a long cached context
+  std::size_t cap_ws_ = 0;
   std::size_t off_cuk_ = 0, off_table_ = 0, off_pos_ = 0, off_slots_ = 0;
 };
 

@@ -50,6 +50,13 @@ SIGNATURES = {
     "paged_prefill_attention": (None, [
         _p, _p, _p, _p, _p, _p, _p, _i64, _i64, _i64, _i64, _i64, _i64, _i64, _i64, _i64,
         ctypes.c_int32, ctypes.c_float, ctypes.c_int, _p]),
+    "paged_prefill_attention_workspace": (None, [
+        _p, _p, _p, _p, _p, _p, _p, _i64, _i64, _i64, _i64, _i64, _i64, _i64, _i64, _i64,
+        ctypes.c_int32, ctypes.c_float, _p, ctypes.c_size_t, ctypes.c_int, _p]),
+    "varlen_prefill_attention_workspace": (None, [
+        _p, _p, _p, _p, _p, _p, _i64, _i64, _i64, _i64, _i64, _i64, _i64, ctypes.c_int32,
+        ctypes.c_float, _p, ctypes.c_size_t, ctypes.c_int, _p]),
+    "prefill_attention_workspace_size": (ctypes.c_size_t, [_i64, _i64, _i64, _i64, _i64, _i64, ctypes.c_int32]),
     "varlen_prefill_attention": (None, [
         _p, _p, _p, _p, _p, _p, _i64, _i64, _i64, _i64, _i64, _i64, _i64, ctypes.c_int32,
         ctypes.c_float, ctypes.c_int, _p]),

@@ -245,22 +245,26 @@ def prefill_attn(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, cu_seqlens_q
     if out is None:
         out = torch.empty_like(q)
     w = -1 if window_left is None else int(window_left)
+    Hkv = k.shape[-2]
+    need = int(L.prefill_attention_workspace_size(B, Hq, Hkv, D, max_seqlen_q, max_seqlen_k, w))
+    workspace = torch.empty(need, dtype=torch.uint8, device=q.device) if need else None
     if block_table is not None:
         NB, BS, Hkv, D2 = k.shape
         if D2 != D or block_table.dtype != torch.int32:
             raise _lib.OxideError("k_cache [NB, BS, Hkv, D] and int32 block_table expected")
         max_blocks = block_table.shape[1] if block_table.dim() == 2 else 0
-        L.paged_prefill_attention(_ptr(out), _ptr(q), _ptr(k), _ptr(v), _ptr(cu_seqlens_q),
-                                  _ptr(cu_seqlens_k), _ptr(block_table), max_blocks, NB, B, Hq, Hkv,
-                                  D, BS, max_seqlen_q, max_seqlen_k, w, float(softmax_scale),
-                                  dtype_code(q.dtype), _stream(q))
+        L.paged_prefill_attention_workspace(_ptr(out), _ptr(q), _ptr(k), _ptr(v), _ptr(cu_seqlens_q),
+                                            _ptr(cu_seqlens_k), _ptr(block_table), max_blocks, NB, B, Hq, Hkv,
+                                            D, BS, max_seqlen_q, max_seqlen_k, w, float(softmax_scale),
+                                            _ptr(workspace), need, dtype_code(q.dtype), _stream(q))
     else:
         Tk, Hkv, D2 = k.shape
         if D2 != D:
             raise _lib.OxideError("k [total_k, Hkv, D] expected")
-        L.varlen_prefill_attention(_ptr(out), _ptr(q), _ptr(k), _ptr(v), _ptr(cu_seqlens_q),
-                                   _ptr(cu_seqlens_k), Tk, B, Hq, Hkv, D, max_seqlen_q, max_seqlen_k,
-                                   w, float(softmax_scale), dtype_code(q.dtype), _stream(q))
+        L.varlen_prefill_attention_workspace(_ptr(out), _ptr(q), _ptr(k), _ptr(v), _ptr(cu_seqlens_q),
+                                             _ptr(cu_seqlens_k), Tk, B, Hq, Hkv, D, max_seqlen_q, max_seqlen_k,
+                                             w, float(softmax_scale), _ptr(workspace), need, dtype_code(q.dtype),
+                                             _stream(q))
     _lib.check()
     return out
 
