@@ -136,6 +136,16 @@ def test_prefill_random_shapes_vs_oracle(device, case):
     assert_attn_close(got, oracle.prefill_attention(q, kc, vc, cuq, cuk, scale, table, window, dtype))
 
 
+# 32 prompts of about one length fill four rounds of the chip's workgroup slots, so that
+# row tiles go in pairs (9 tiles, the middle one alone; shorter prompts of 8); a ragged
+# batch of the same grid takes them one by one.
+@pytest.mark.parametrize("lens", [[288, 257, 256, 225] * 8, [288, 1, 33, 0] * 8], ids=["pairs", "ragged"])
+def test_prefill_many_prompts_vs_oracle(device, lens):
+    q, kc, vc, cuq, cuk, table = _case(61, lens, lens, 32, 8, 64, 256)
+    got = to_f32(_gpu(device, q, kc, vc, cuq, cuk, table, 0.125, -1, "bf16"))
+    assert_attn_close(got, oracle.prefill_attention(q, kc, vc, cuq, cuk, 0.125, table, -1, "bf16"))
+
+
 # Queries behind long cached contexts, whose keys are split over workgroups: the piece
 # and tile edges, sequences with nothing to split or no queries, the smallest batch and
 # the largest that is split (64), rows of 128 that groups of 7 and 5 do not fill.

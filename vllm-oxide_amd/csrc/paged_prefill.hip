@@ -37,8 +37,9 @@
 // Workgroup order is XCD-aware: all row tiles of one (sequence, kv head) run
 // on one XCD (workgroup i runs on XCD i % 8), so its K/V is fetched from HBM
 // once into that XCD's L2 and re-read from there; within a unit the tiles
-// with the most keys (last tokens) start first.  For short prompts (kPair) a
-// workgroup takes two row tiles of its unit, n - 1 - i and then i.
+// with the most keys (last tokens) start first.  In large batches of short prompts of
+// about one length (kPair) a workgroup takes two row tiles of its unit, n - 1 - i and
+// then i; behind long cached contexts (kSplit) a row tile's keys are cut into pieces.
 #include <math.h>
 
 #include <algorithm>
@@ -93,7 +94,7 @@ struct PrefillParams {
   int shared_hint;
   int dec_batch;
   int* shared_out;  // the number of shared blocks found (written by workgroup 0)
-  int pair;         // 1: each workgroup takes row tiles n - 1 - i and then i of its unit
+  int pair;         // 1: the kPair instances
   // Balanced launch (kernel instances with kSplit): the most pieces it cuts, and the
   // batch size.  Partial rows go to part_o / part_lse, row piece * kPfRows + row.
   int max_pieces;
@@ -267,10 +268,18 @@ __global__ __launch_bounds__(kPfThreads, 2) void paged_prefill_attn(PrefillParam
   // Balanced launch: XCD x takes the x-th eighth of the pieces.
   const int i = blockIdx.x;
   const int j = i / kPfXcds;
-  const int wpu = kPair ? (p.tiles_per_unit + 1) / 2 : p.tiles_per_unit;  // workgroups per unit
-  const int u = (j / wpu) * kPfXcds + i % kPfXcds;
+  const int u = (j / p.tiles_per_unit) * kPfXcds + i % kPfXcds;
   if (!kSplit && u >= p.units) return;
-  const int jj = j % wpu;
+  const int jj = j % p.tiles_per_unit;
+  // kPair: a workgroup takes row tiles n - 1 - jj and then jj (half of the workgroups
+  // end at once) where the prompts are of about one length; in ragged batches the pairs
+  // would be uneven.
+  bool pair = false;
+  if constexpr (kPair) {
+    const int64_t total = static_cast<int64_t>(p.cu_seqlens_q[p.batch]) - p.cu_seqlens_q[0];
+    pair = 4 * total >= 3 * static_cast<int64_t>(p.batch) * p.max_seqlen_q;
+    if (pair && jj >= (p.tiles_per_unit + 1) / 2) return;
+  }
   for (int pass = 0; pass < (kPair ? 2 : 1); ++pass) {
   int tile, b, kh, split = 0;
   int piece = 0, s0 = 0, s1 = 0;  // kSplit: the piece and its steps of the tile
@@ -296,7 +305,7 @@ __global__ __launch_bounds__(kPfThreads, 2) void paged_prefill_attn(PrefillParam
   } else {
     tile = pass == 0 ? p.tiles_per_unit - 1 - jj : jj;
     if (pass == 1) {
-      if (tile >= p.tiles_per_unit - 1 - jj) break;  // the middle tile of an odd count: done
+      if (!pair || tile >= p.tiles_per_unit - 1 - jj) break;  // (the middle tile of an odd count: done)
       __syncthreads();  // the previous tile's last LDS reads before this tile's first loads
     }
     b = kPrefix ? 0 : u / p.num_kv_heads;
@@ -856,7 +865,7 @@ bool launch_prefill(const PrefillParams& p, int head_dim, hipStream_t s) {
     return true;
   }
   const int64_t units8 = ceil_div64(p.units, kPfXcds) * kPfXcds;
-  const dim3 grid(static_cast<unsigned>(units8 * (p.pair ? (p.tiles_per_unit + 1) / 2 : p.tiles_per_unit)));
+  const dim3 grid(static_cast<unsigned>(units8 * p.tiles_per_unit));
   if (head_dim == 128) {
     launch_mode<Tag, 128>(p, grid, s);
     return true;
@@ -935,13 +944,17 @@ void prefill_impl(void* out, const void* q, const void* k, const void* v, const 
   }
   p.tiles_per_unit = static_cast<int>(tiles);
   p.units = static_cast<int>(units);
-  // Short prompts with no cached prefix: a workgroup takes a unit's row tiles n - 1 - i
-  // and then i (a separate kernel instance), the same keys per workgroup and half the
-  // workgroup starts.  Measured on MI355X, Qwen3-8B heads, bit-identical output:
-  // 16 x 1024 212.1 -> 202.8 us, 32 x 512 138.6 -> 135.7 us, 8 x 2048 324.2 -> 319.9 us;
-  // for 4 x 4096 and 1 x 8192 pairing measured +0.7 / +1.3 %, and with a cached prefix
-  // the tiles already carry equal keys.
-  p.pair = (tiles >= 2 && max_seqlen_k <= max_seqlen_q && max_seqlen_q <= 2048) ? 1 : 0;
+  // Prompts with no cached prefix, of at most 2048 tokens and about one length (the
+  // kernel looks), with work for four rounds of the chip's slots: a workgroup takes a
+  // unit's row tiles n - 1 - i and then i (a separate kernel instance), the same keys per
+  // workgroup and half the workgroup starts.  Single -> paired: 32 x 512 (G = 2) 69.0 ->
+  // 62.7 us, 16 x 1024 188 -> 184, 8 x 2048 303 -> 296; smaller or ragged batches lose
+  // (1 x 300 11.6 -> 17.0, 128 x 128 51 -> 62, 8 of 200-1000 81 -> 89), and so do 4 x
+  // 4096 and prompts behind a cached prefix, whose tiles already carry equal keys.
+  p.pair = (tiles >= 8 && max_seqlen_k <= max_seqlen_q && max_seqlen_q <= 2048 &&
+            tiles * units >= 8 * static_cast<int64_t>(oxide::device_cu_count()))
+               ? 1
+               : 0;
   p.block_size = static_cast<int>(block_table ? page_block_size : 1);
   p.window_left = window_left < 0 ? -1 : window_left;
   p.scale_log2 = softmax_scale * 1.4426950408889634f;
