@@ -96,6 +96,30 @@ def test_decode_vs_oracle(device, case, decode_path):
             assert not got[b].any()
 
 
+# Few (query head, sequence) pairs with many splits: the merge's 16 waves (from 96 splits
+# on), more splits than one round of its loads holds (256), and short, single-split and
+# empty sequences beside a long one.
+MANY_SPLITS = [
+    # (B, Hq, Hkv, D, BS, NB, lens, window, dtype)
+    (1, 2, 1, 64, 64, 200, [96 * 128], -1, "bf16"),
+    (5, 4, 2, 128, 256, 60, [95 * 128 + 1, 128, 129, 0, 1], -1, "f16"),
+    (1, 4, 1, 64, 256, 140, [33333], -1, "bf16"),
+    (2, 8, 1, 128, 256, 80, [14000, 3000], 12500, "bf16"),
+]
+
+
+@pytest.mark.parametrize("case", MANY_SPLITS, ids=[f"m{i}" for i in range(len(MANY_SPLITS))])
+def test_decode_many_splits_vs_oracle(device, case):
+    import oxide_paged_kv as ox
+
+    B, Hq, Hkv, D, BS, NB, lens, window, dtype = case
+    assert ox.split_tokens(B, Hkv, max(lens)) == 128 and B * Hq <= 64 and max(lens) > 95 * 128
+    q, kc, vc, cu, table, mx = _case(13, B, Hq, Hkv, D, BS, NB, lens, dtype)
+    print(f"decode many splits B={B} Hq={Hq} Hkv={Hkv} D={D} lens={lens} window={window} {dtype}", flush=True)
+    got = to_f32(_run(device, q, kc, vc, cu, table, mx, 1.0 / math.sqrt(D), window, dtype))
+    assert_attn_close(got, oracle.paged_decode_attention(q, kc, vc, cu, table, 1.0 / math.sqrt(D), window, dtype))
+
+
 def _random_shapes(seed, n):
     """Seeded random shapes over what the fixed cases combine separately: kv heads
     1/2/3/4/8, groups 1-8 and 16, D 64/128, page sizes 16/32/256, bf16/f16, ragged

@@ -695,19 +695,19 @@ __global__ __launch_bounds__(64 * kStreamWaves, 1) void paged_decode_stream(Deco
   }
 }
 
-// Pass 2: one workgroup of 4 waves per (query head, sequence) merges the
+// Pass 2: one workgroup of kMergeWaves waves per (query head, sequence) merges the
 // splits that intersect [lo, L) with log-sum-exp weights; each wave takes a
-// contiguous quarter of the splits and the quarters are combined in LDS.
+// contiguous share of the splits and the shares are combined in LDS.
 // Sequences with a single split were finished by pass 1 and are skipped;
 // empty sequences get zeros.  A wave's log2-sum-exps and the partial rows of its
 // first kChunk splits are loaded in one round (clamped indices; weights select
 // the extra rows away), so the merge is two dependent rounds of loads after the
 // lengths, not three.
-template <class Tag, int D, int kChunk = 8>
-__global__ __launch_bounds__(kThreads) void paged_decode_merge(DecodeParams p) {
+template <class Tag, int D, int kMergeWaves, int kChunk>
+__global__ __launch_bounds__(64 * kMergeWaves) void paged_decode_merge(DecodeParams p) {
   constexpr int PER = D / 64;
-  __shared__ float s_o[kWaves][D];
-  __shared__ float s_mw[kWaves][2];
+  __shared__ float s_o[kMergeWaves][D];
+  __shared__ float s_mw[kMergeWaves][2];
   const int h = blockIdx.x;
   const int b = blockIdx.y;
   const int wave = threadIdx.x >> 6;
@@ -715,7 +715,7 @@ __global__ __launch_bounds__(kThreads) void paged_decode_merge(DecodeParams p) {
   const int L = seq_len(p, b);
   uint16_t* out = static_cast<uint16_t*>(p.out) + (static_cast<int64_t>(b) * p.num_heads + h) * D;
   if (L == 0) {
-    for (int i = threadIdx.x; i < D; i += kThreads) out[i] = 0;
+    for (int i = threadIdx.x; i < D; i += 64 * kMergeWaves) out[i] = 0;
     // Fused append of a sequence with no keys to attend to: the first query
     // head of each kv-head group writes that head's slice of the new row.
     const int G = p.num_heads / p.num_kv_heads;
@@ -724,7 +724,7 @@ __global__ __launch_bounds__(kThreads) void paged_decode_merge(DecodeParams p) {
       const int kh = h / G;
       const int64_t row_stride = static_cast<int64_t>(p.num_kv_heads) * D;
       const int64_t src = (static_cast<int64_t>(b) * p.num_kv_heads + kh) * D;
-      for (int i = threadIdx.x; slot >= 0 && i < D; i += kThreads) {
+      for (int i = threadIdx.x; slot >= 0 && i < D; i += 64 * kMergeWaves) {
         const_cast<uint16_t*>(static_cast<const uint16_t*>(p.k))[slot * row_stride + kh * D + i] =
             static_cast<const uint16_t*>(p.new_k)[src + i];
         const_cast<uint16_t*>(static_cast<const uint16_t*>(p.v))[slot * row_stride + kh * D + i] =
@@ -738,7 +738,7 @@ __global__ __launch_bounds__(kThreads) void paged_decode_merge(DecodeParams p) {
   const int last = (L - 1) / p.split_tokens;
   if (first == last) return;
   const int n = last - first + 1;
-  const int chunk = (n + kWaves - 1) / kWaves;
+  const int chunk = (n + kMergeWaves - 1) / kMergeWaves;
   const int w_first = first + wave * chunk;
   const int w_last = min(last, w_first + chunk - 1);
 
@@ -804,11 +804,11 @@ __global__ __launch_bounds__(kThreads) void paged_decode_merge(DecodeParams p) {
   if (wave == 0) {
     float Mt = -INFINITY;
 #pragma unroll
-    for (int w = 0; w < kWaves; ++w) Mt = fmaxf(Mt, s_mw[w][0]);
+    for (int w = 0; w < kMergeWaves; ++w) Mt = fmaxf(Mt, s_mw[w][0]);
     const float mt = Mt == -INFINITY ? 0.f : Mt;
-    float f[kWaves], wt = 0.f;
+    float f[kMergeWaves], wt = 0.f;
 #pragma unroll
-    for (int w = 0; w < kWaves; ++w) {
+    for (int w = 0; w < kMergeWaves; ++w) {
       const float mw = s_mw[w][0];
       f[w] = mw == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(mw - mt);
       wt += f[w] * s_mw[w][1];
@@ -818,7 +818,7 @@ __global__ __launch_bounds__(kThreads) void paged_decode_merge(DecodeParams p) {
     for (int k = 0; k < PER; ++k) {
       float acc = 0.f;
 #pragma unroll
-      for (int w = 0; w < kWaves; ++w) acc = fmaf(f[w], s_o[w][lane + 64 * k], acc);
+      for (int w = 0; w < kMergeWaves; ++w) acc = fmaf(f[w], s_o[w][lane + 64 * k], acc);
       out[lane + 64 * k] = pack1(Tag{}, acc * inv);
     }
   }
@@ -1207,6 +1207,20 @@ bool dispatch_group(const DecodeParams& p, int64_t batch, int group, hipStream_t
   }
 }
 
+// Many splits of few (query head, sequence) pairs: 16 waves share a pair's splits, 16
+// rows in flight each, so that up to 256 splits take one round of loads where four waves
+// walked them in eight.  Per call, 4 -> 16 waves: one sequence of 32k keys (256 splits,
+// 32 heads) 32.9 -> 31.2 us, with 28 heads over 4 kv heads 25.1 -> 23.1, 128k 105.4 ->
+// 99.4.  With fewer splits or more pairs the larger workgroups lose: one of 8k (64
+// splits) 12.8 -> 13.9, 4 of 4k-16k (128 splits, 128 pairs) 45.1 -> 46.2.
+template <class Tag, int D>
+void launch_split_merge(const DecodeParams& p, dim3 grid, hipStream_t s) {
+  if (p.max_splits >= 96 && p.num_heads * p.batch <= 64)
+    hipLaunchKernelGGL((paged_decode_merge<Tag, D, 16, 16>), grid, dim3(1024), 0, s, p);
+  else
+    hipLaunchKernelGGL((paged_decode_merge<Tag, D, 4, 8>), grid, dim3(256), 0, s, p);
+}
+
 // Workgroups per CU of the persistent path, at most (bounds the workspace).
 constexpr int kMaxWgsPerCu = 4;
 constexpr int kMaxDevices = 64;
@@ -1340,12 +1354,12 @@ bool dispatch(const DecodeParams& p, int64_t batch, int head_dim, int group, hip
   const dim3 mgrid(static_cast<unsigned>(p.num_heads), static_cast<unsigned>(batch));
   if (head_dim == 128) {
     if (!dispatch_group<Tag, 128>(p, batch, group, s)) return false;
-    hipLaunchKernelGGL((paged_decode_merge<Tag, 128>), mgrid, dim3(kThreads), 0, s, p);
+    launch_split_merge<Tag, 128>(p, mgrid, s);
     return true;
   }
   if (head_dim == 64) {
     if (!dispatch_group<Tag, 64>(p, batch, group, s)) return false;
-    hipLaunchKernelGGL((paged_decode_merge<Tag, 64>), mgrid, dim3(kThreads), 0, s, p);
+    launch_split_merge<Tag, 64>(p, mgrid, s);
     return true;
   }
   return false;
