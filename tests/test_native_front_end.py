@@ -1,0 +1,108 @@
+"""The ops' native front end (_native.so) against the general Python code it stands in for:
+the same outputs bit for bit over the argument forms it takes and those it leaves, and the
+same errors."""
+import math
+
+import numpy as np
+import pytest
+import torch
+
+import oxide_paged_kv as ox
+from oxide_paged_kv import ops
+
+
+def _general(monkeypatch):
+    """ops with the native front end declining every call."""
+    class Declines:
+        def __getattr__(self, name):
+            return lambda *args: None
+
+    monkeypatch.setattr(ops, "_native", Declines())
+
+
+def _inputs(device, dtype=torch.bfloat16, B=3, Hq=8, Hkv=4, D=128, BS=64):
+    g = torch.Generator(device="cpu").manual_seed(3)
+    rnd = lambda *s: torch.randn(s, generator=g).to(dtype).to(device)  # noqa: E731
+    lens = torch.tensor([70, 1, 130], dtype=torch.int32)
+    table = torch.tensor([[2, 5, 0], [1, 0, 0], [7, 3, 4]], dtype=torch.int32)
+    cu = torch.zeros(B + 1, dtype=torch.int32)
+    cu[1:] = torch.cumsum(lens, 0)
+    slots = torch.tensor([5 * BS + 5, BS, 4 * BS + 1], dtype=torch.int64)
+    return {"q": rnd(B, Hq, D), "k": rnd(8, BS, Hkv, D), "v": rnd(8, BS, Hkv, D), "key": rnd(B, Hkv, D),
+            "value": rnd(B, Hkv, D), "qkv": rnd(B, (Hq + 2 * Hkv) * D), "w": rnd(D), "cu": cu.to(device),
+            "lens": lens.to(device), "table": table.to(device), "slots": slots.to(device),
+            "rope": ox.rope_cos_sin_cache(256, D, device=device), "pos": (lens - 1).to(device), "BS": BS}
+
+
+def _calls(s):
+    """The calls of a step, in the forms the native code takes and in others."""
+    BS, sc = s["BS"], 1 / math.sqrt(128)
+    out = []
+    for window, append, cu, scale in ((None, None, s["cu"], sc), (50, None, s["cu"].view(torch.uint32), sc),
+                                      (None, (s["key"], s["value"], s["slots"]), s["cu"], sc),
+                                      (None, [s["key"], s["value"], s["slots"]], s["cu"], np.float64(sc))):
+        k, v = s["k"].clone(), s["v"].clone()
+        out += [ox.decode_attn(s["q"], k, v, cu, s["table"], 130, scale, window_left=window, page_block_size=BS,
+                               append=append), k, v]
+    given, ws = torch.empty_like(s["q"]), torch.empty(1 << 22, dtype=torch.uint8, device=s["q"].device)
+    r = ox.decode_attn(s["q"], s["k"], s["v"], s["cu"], s["table"], 130, sc, page_block_size=BS, out=given,
+                       workspace=ws)
+    assert r is given
+    out.append(r.clone())
+    cq = torch.tensor([0, 1, 2, 3], dtype=torch.int32, device=s["q"].device)
+    rows = s["k"].reshape(-1, *s["k"].shape[2:])
+    for window in (None, 40):
+        out.append(ox.prefill_attn(s["q"], s["k"], s["v"], cq, s["cu"], 1, 130, sc, s["table"], window))
+        out.append(ox.prefill_attn(s["q"], rows, s["v"].reshape(rows.shape), cq, s["cu"], 1, 130, sc,
+                                   window_left=window))
+    for w, slots in ((s["w"], s["slots"]), (None, None)):
+        k, v = s["k"].clone(), s["v"].clone()
+        cache = (k, v, slots) if slots is not None else (None, None, None)
+        out += [ox.qk_norm_rope_and_cache(s["qkv"], 8, 4, w, w, 1e-6, s["rope"], s["pos"], *cache), k, v]
+    out.append(ox.qk_norm_rope_and_cache(s["qkv"], 8, 4, s["w"], s["w"], 1e-6, s["rope"], s["pos"], return_k=True)[1])
+    return out + list(ox.build_decode_metadata(s["lens"], s["table"], BS))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "f16"])
+def test_native_calls_equal_general_calls(device, dtype, monkeypatch):
+    print(f"native front end {dtype}", flush=True)
+    got = _calls(_inputs(device, dtype))
+    _general(monkeypatch)
+    want = _calls(_inputs(device, dtype))
+    torch.cuda.synchronize()
+    assert len(got) == len(want)
+    for g, w in zip(got, want):
+        assert g.dtype == w.dtype and g.shape == w.shape and torch.equal(g, w)
+
+
+@pytest.mark.gpu
+def test_library_errors_raise_through_the_native_calls(device):
+    """Errors the library records (a workspace-free shape check here: head size 96)."""
+    q = torch.zeros(1, 4, 96, dtype=torch.bfloat16, device=device)
+    k = torch.zeros(2, 64, 2, 96, dtype=torch.bfloat16, device=device)
+    i32 = lambda *v: torch.tensor(v, dtype=torch.int32, device=device)  # noqa: E731
+    for _ in range(2):  # the error is cleared when it is raised
+        with pytest.raises(ox.OxideError):
+            ox.decode_attn(q, k, k, i32(0, 5), i32(0)[None], 5, 0.1, page_block_size=64)
+        with pytest.raises(ox.OxideError):
+            ox.prefill_attn(q, k, k, i32(0, 1), i32(0, 5), 1, 5, 0.1, i32(0)[None])
+
+
+def test_host_tensors_are_refused_alike(monkeypatch):
+    s = _inputs("cpu")
+    calls = [lambda: ox.decode_attn(s["q"], s["k"], s["v"], s["cu"], s["table"], 130, 0.1, page_block_size=64),
+             lambda: ox.decode_attn(s["q"], s["k"], s["v"], s["cu"], s["table"], 130, 0.1, page_block_size=32),
+             lambda: ox.decode_attn(s["q"], s["k"].float(), s["v"], s["cu"], s["table"], 130, 0.1, page_block_size=64),
+             lambda: ox.prefill_attn(s["q"], s["k"], s["v"], s["cu"], s["cu"], 1, 130, 0.1, s["table"]),
+             lambda: ox.qk_norm_rope_and_cache(s["qkv"], 8, 4, None, None, 1e-6, s["rope"], s["pos"].long()),
+             lambda: ox.build_decode_metadata(s["lens"].long(), s["table"], 64)]
+    messages = []
+    for general in (False, True):
+        if general:
+            _general(monkeypatch)
+        for call in calls:
+            with pytest.raises(ox.OxideError) as e:
+                call()
+            messages.append(str(e.value))
+    assert messages[:len(calls)] == messages[len(calls):]

@@ -24,6 +24,9 @@ INCLUDE = REPO / "include"
 BUILD = PKG / "_build"
 LIB = PKG / "liboxide_paged_kv.so"
 STATIC_LIB = PKG / "liboxide_paged_kv.a"
+# The Python ops' native front end: a CPython module against torch's C++ headers.
+NATIVE_SRC = PKG / "pyext" / "native_ops.cpp"
+NATIVE_LIB = PKG / "oxide_paged_kv" / "_native.so"
 HOST_TEST_SRC = REPO / "tests" / "cpp" / "test_host.cpp"
 HOST_TEST_BIN = REPO / "tests" / "cpp" / "build" / "test_host"
 HOST_TEST_STAMP = HOST_TEST_BIN.with_suffix(".sources.sha256")
@@ -76,11 +79,32 @@ def _compile(src: Path):
     return obj, _parse_resources(r.stderr)
 
 
+def build_native() -> Path:
+    """oxide_paged_kv/_native.so with the host compiler; it links torch's libraries, which
+    `import torch` has loaded by then."""
+    import sysconfig
+
+    import torch
+
+    t = Path(torch.__file__).resolve().parent
+    cmd = ["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
+           f"-D_GLIBCXX_USE_CXX11_ABI={int(torch.compiled_with_cxx11_abi())}", "-I", str(INCLUDE),
+           "-isystem", str(t / "include"), "-isystem", str(t / "include" / "torch" / "csrc" / "api" / "include"),
+           "-isystem", "/opt/rocm/include", "-isystem", sysconfig.get_paths()["include"], str(NATIVE_SRC),
+           "-o", str(NATIVE_LIB), "-L", str(t / "lib"), "-ltorch_python", "-ltorch_cpu", "-lc10", "-lc10_hip"]
+    r = subprocess.run(cmd, capture_output=True, text=True)
+    if r.returncode != 0:
+        raise RuntimeError(f"g++ failed for {NATIVE_SRC.name}:\n{r.stdout}\n{r.stderr}")
+    return NATIVE_LIB
+
+
 def build(verbose: bool = False) -> Path:
     BUILD.mkdir(exist_ok=True)
     srcs = _sources()
-    with ThreadPoolExecutor(max_workers=min(8, len(srcs))) as ex:
+    with ThreadPoolExecutor(max_workers=min(9, len(srcs) + 1)) as ex:
+        native = ex.submit(build_native)
         results = list(ex.map(_compile, srcs))
+        native.result()
     objs = [o for o, _ in results]
     import json
 

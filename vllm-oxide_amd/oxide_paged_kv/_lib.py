@@ -8,6 +8,8 @@ import ctypes
 import os
 from pathlib import Path
 
+import torch  # noqa: F401  (its libraries first: _native links to them)
+
 PKG_DIR = Path(__file__).resolve().parent.parent
 # OXIDE_PAGED_KV_LIB points at another build of the same library (e.g. a tuning variant).
 LIB_PATH = Path(os.environ.get("OXIDE_PAGED_KV_LIB", PKG_DIR / "liboxide_paged_kv.so"))
@@ -91,6 +93,11 @@ def load() -> ctypes.CDLL:
             fn = getattr(L, name)
             fn.restype = res
             fn.argtypes = args
+        # The native front end (_native.so, built beside the library) calls this library.
+        from . import _native
+
+        for name in SIGNATURES:
+            _native.bind(name, ctypes.cast(getattr(L, name), ctypes.c_void_p).value)
         _lib = L
     return _lib
 

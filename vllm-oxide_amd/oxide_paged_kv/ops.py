@@ -11,12 +11,15 @@
 
 Tensors must be contiguous CUDA (HIP) tensors; every call goes to the HIP library
 on torch's current stream and raises OxideError if the library reports an error.
+The calls of a serving step (decode, prefill, prologue, metadata) go through the native
+front end (_native.so, pyext/native_ops.cpp) when their arguments are of the plain form;
+the code here handles the other forms and raises the argument errors.
 """
 from __future__ import annotations
 
 import torch
 
-from . import _lib
+from . import _lib, _native
 
 _DTYPE_CODE = {torch.float16: _lib.DTYPE_F16, torch.bfloat16: _lib.DTYPE_BF16,
                torch.float32: _lib.DTYPE_F32}
@@ -160,6 +163,11 @@ def decode_attn(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor,
     "auto" goes through paged_decode_attention_shared_prefix_mode.
     """
     L = _lib.load()
+    if (path == 0 or path == "auto") and not noalloc and shared_prefix_blocks is None:
+        r = _native.decode(q, k_cache, v_cache, cu_seqlens_k, block_table, max_seqlen_k, softmax_scale, window_left,
+                           page_block_size, out, workspace, append)
+        if r is not None:
+            return r if r is not False else _lib.check()
     B, Hq, D = q.shape
     NB, BS, Hkv, D2 = k_cache.shape
     if D2 != D or BS != page_block_size or v_cache.shape != k_cache.shape:
@@ -233,6 +241,10 @@ def prefill_attn(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, cu_seqlens_q
     cu_seqlens_k are 32-bit [B + 1] (uint32 bits).  window_left None = unbounded.
     """
     L = _lib.load()
+    r = _native.prefill(q, k, v, cu_seqlens_q, cu_seqlens_k, max_seqlen_q, max_seqlen_k, softmax_scale, block_table,
+                        window_left, out)
+    if r is not None:
+        return r if r is not False else _lib.check()
     Tq, Hq, D = q.shape
     if cu_seqlens_q.dtype not in (torch.int32, torch.uint32) or \
             cu_seqlens_k.dtype not in (torch.int32, torch.uint32):
@@ -296,6 +308,11 @@ def qk_norm_rope_and_cache(qkv: torch.Tensor, num_heads: int, num_kv_heads: int,
     serving loop reuses its buffers); k_out implies return_k.
     """
     L = _lib.load()
+    if not return_k and k_out is None:
+        r = _native.prologue(qkv, num_heads, num_kv_heads, q_norm_weight, k_norm_weight, eps, cos_sin_cache, positions,
+                             key_cache, value_cache, slot_mapping, q_out)
+        if r is not None:
+            return r if r is not False else _lib.check()
     T = qkv.shape[0]
     D = cos_sin_cache.shape[1]
     if positions.dtype != torch.int32 or cos_sin_cache.dtype != torch.float32:
@@ -325,6 +342,9 @@ def build_decode_metadata(context_lens: torch.Tensor, block_table: torch.Tensor,
     slot_mapping int64 [B]) from context_lens (int32 bits of uint32, [B]) and the
     0-padded int32 block table [B, max_blocks]."""
     L = _lib.load()
+    r = _native.metadata(context_lens, block_table, block_size)
+    if r is not None:
+        return r if r is not False else _lib.check()
     if context_lens.dtype not in (torch.int32, torch.uint32) or block_table.dtype != torch.int32:
         raise _lib.OxideError("context_lens must be 32-bit and block_table int32")
     B = context_lens.shape[0]
