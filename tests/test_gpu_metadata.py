@@ -33,6 +33,12 @@ def test_device_metadata_matches_oracle(device, B, bs, seed):
     assert np.array_equal(slots.cpu().numpy(), want_slots)
 
 
+@pytest.mark.parametrize("B", [63, 65, 1024, 1025])
+def test_device_metadata_wave_and_workgroup_edges(device, B):
+    """A lane per sequence: one wave, a second one, the full workgroup, runs of two."""
+    test_device_metadata_matches_oracle(device, B, 16, B)
+
+
 def test_device_metadata_reference_decode_vectors(device):
     """metadata.rs:94-103 (context lens 5, 20, 3 -> cu 0,5,25,28) with tables whose
     new-token slots follow kv_cache_manager.rs's formula."""

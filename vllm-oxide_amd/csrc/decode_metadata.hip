@@ -12,9 +12,12 @@
 // engine that keeps context lengths and block tables on the device can run
 // this once per step and feed every layer's append and attention from it.
 //
-// One workgroup of 1024 lanes: each lane sums a contiguous run of sequences,
-// the run totals are scanned in LDS, and each lane writes its run's prefix
-// sums and slots.  Batches of up to 65535 sequences.
+// One workgroup, a lane per sequence up to 1024 of them: each lane sums a contiguous
+// run of sequences, the run totals are scanned -- inside the waves by shuffles, the
+// waves' totals through LDS -- and each lane writes its run's prefix sums and slots.
+// Batches of up to 65535 sequences.  Its time is latency (the lengths, then the table
+// entries they select, and the scan): 3.2 -> 1.9 us at 4 sequences against a scan of
+// 1024 lanes through LDS with two barriers a step.
 #include "oxide_common.hpp"
 
 namespace {
@@ -27,23 +30,25 @@ __global__ __launch_bounds__(kLanes) void decode_metadata_kernel(const uint32_t*
                                                                  int block_size,
                                                                  uint32_t* __restrict__ cu_seqlens_k,
                                                                  int64_t* __restrict__ slot_mapping) {
-  __shared__ uint32_t s_sum[kLanes];
+  __shared__ uint32_t s_wave[kLanes / 64];
   const int t = threadIdx.x;
-  const int per = (batch + kLanes - 1) / kLanes;
+  const int per = (batch + blockDim.x - 1) / blockDim.x;
   const int b0 = t * per;
   const int b1 = min(batch, b0 + per);
   uint32_t run = 0;
   for (int b = b0; b < b1; ++b) run += context_lens[b];
-  s_sum[t] = run;
-  __syncthreads();
-  // Inclusive Hillis-Steele scan of the run totals.
-  for (int off = 1; off < kLanes; off <<= 1) {
-    const uint32_t add = t >= off ? s_sum[t - off] : 0u;
-    __syncthreads();
-    s_sum[t] += add;
-    __syncthreads();
+  uint32_t acc = run;  // inclusive over the wave's runs
+#pragma unroll
+  for (int off = 1; off < 64; off <<= 1) {
+    const uint32_t add = __shfl_up(acc, off);
+    if ((t & 63) >= off) acc += add;
   }
-  uint32_t acc = s_sum[t] - run;  // exclusive prefix of this run
+  acc -= run;  // exclusive
+  if (blockDim.x > 64) {
+    if ((t & 63) == 63) s_wave[t >> 6] = acc + run;
+    __syncthreads();
+    for (int w = 0; w < t >> 6; ++w) acc += s_wave[w];
+  }
   if (t == 0) cu_seqlens_k[0] = 0;
   for (int b = b0; b < b1; ++b) {
     const uint32_t L = context_lens[b];
@@ -51,11 +56,11 @@ __global__ __launch_bounds__(kLanes) void decode_metadata_kernel(const uint32_t*
     cu_seqlens_k[b + 1] = acc;
     int64_t slot = -1;
     if (L > 0) {
-      const int64_t pos = static_cast<int64_t>(L) - 1;
-      const int64_t blk = pos / block_size;
+      const uint32_t bs = static_cast<uint32_t>(block_size);
+      const uint32_t blk = (L - 1) / bs;
       if (blk < max_blocks)
         slot = static_cast<int64_t>(block_table[static_cast<int64_t>(b) * max_blocks + blk]) * block_size +
-               pos % block_size;
+               (L - 1) % bs;
     }
     slot_mapping[b] = slot;
   }
@@ -77,7 +82,8 @@ extern "C" void build_decode_metadata_device(const uint32_t* context_lens, const
     oxide::set_error(OXIDE_ERR_INVALID_ARGUMENT);
     return;
   }
-  hipLaunchKernelGGL(decode_metadata_kernel, dim3(1), dim3(kLanes), 0, oxide::as_stream(stream),
+  const int lanes = batch >= kLanes ? kLanes : static_cast<int>((batch + 63) / 64 * 64);
+  hipLaunchKernelGGL(decode_metadata_kernel, dim3(1), dim3(lanes > 0 ? lanes : 64), 0, oxide::as_stream(stream),
                      context_lens, block_table, max_blocks_per_seq, static_cast<int>(batch),
                      static_cast<int>(block_size), cu_seqlens_k, slot_mapping);
   oxide::check_launch();
