@@ -495,6 +495,24 @@ def test_decode_fused_append_equals_append_then_attend(device, case, decode_path
     assert np.array_equal(to_bits(v2), to_bits(v1))
 
 
+# Contexts of at most 128 / 256 keys: one split per sequence and no merge, empty
+# sequences (their zeros and their append) included.
+SINGLE_SPLIT = [
+    (5, 16, 8, 128, 256, 20, [0, 10, 0, 256, 129], -1, "bf16"),
+    (4, 28, 4, 64, 16, 80, [128, 1, 0, 127], -1, "f16"),
+    (3, 16, 2, 128, 32, 40, [250, 3, 0], 20, "bf16"),
+]
+
+
+@pytest.mark.parametrize("case", SINGLE_SPLIT, ids=[f"s{i}" for i in range(len(SINGLE_SPLIT))])
+def test_decode_single_split(device, case):
+    import oxide_paged_kv as ox
+
+    assert ox.split_tokens(case[0], case[2], max(case[6])) >= max(case[6])
+    test_decode_vs_oracle(device, case, 1)
+    test_decode_fused_append_equals_append_then_attend(device, case, 1)
+
+
 @pytest.mark.parametrize("cfg_id,path", [(3, 0), (4, 0), (5, 0), (3, 4), (4, 4)],
                          ids=["cfg3", "cfg4", "cfg5", "cfg3-rows", "cfg4-rows"])
 def test_decode_fused_append_full_size(device, cfg_id, path):

@@ -331,6 +331,26 @@ __device__ __forceinline__ void decode_wave_tiles(const DecodeParams& p, char* s
                                           slot_new);
 }
 
+// A sequence without keys: zeros for query heads h0 .. h0 + n - 1, and, with the fused
+// append, the new row's slice of each kv head whose first query head is among them.
+template <int D>
+__device__ __forceinline__ void empty_sequence(const DecodeParams& p, int b, int h0, int n, int threads) {
+  uint16_t* out = static_cast<uint16_t*>(p.out) + (static_cast<int64_t>(b) * p.num_heads + h0) * D;
+  for (int i = threadIdx.x; i < n * D; i += threads) out[i] = 0;
+  const int G = p.num_heads / p.num_kv_heads;
+  if (p.new_k == nullptr || h0 % G != 0) return;
+  const int64_t slot = p.slot_mapping[b];
+  const int kh = h0 / G;
+  const int64_t row_stride = static_cast<int64_t>(p.num_kv_heads) * D;
+  const int64_t src = (static_cast<int64_t>(b) * p.num_kv_heads + kh) * D;
+  for (int i = threadIdx.x; slot >= 0 && i < D; i += threads) {
+    const_cast<uint16_t*>(static_cast<const uint16_t*>(p.k))[slot * row_stride + kh * D + i] =
+        static_cast<const uint16_t*>(p.new_k)[src + i];
+    const_cast<uint16_t*>(static_cast<const uint16_t*>(p.v))[slot * row_stride + kh * D + i] =
+        static_cast<const uint16_t*>(p.new_v)[src + i];
+  }
+}
+
 // Merges the 4 waves' states through LDS and writes, per query q of the group,
 // either the bf16/f16 output row (direct) or the normalised partial o and its
 // log2-sum-exp at partial row prow_base + q * prow_qstride.  Ends with a
@@ -405,6 +425,10 @@ __global__ __launch_bounds__(kThreads) void paged_decode_split(DecodeParams p) {
   const int L = seq_len(p, b);
   const int lo = p.window_left >= 0 ? max(0, L - 1 - p.window_left) : 0;
   const int s0 = split * (kWaves * S::WT);
+  if (p.max_splits == 1 && L == 0) {  // no merge follows
+    empty_sequence<D>(p, b, kh * G, G, kThreads);
+    return;
+  }
   if (s0 >= L || s0 + kWaves * S::WT <= lo) return;
 
   const int wave = threadIdx.x >> 6;
@@ -715,22 +739,7 @@ __global__ __launch_bounds__(64 * kMergeWaves) void paged_decode_merge(DecodePar
   const int L = seq_len(p, b);
   uint16_t* out = static_cast<uint16_t*>(p.out) + (static_cast<int64_t>(b) * p.num_heads + h) * D;
   if (L == 0) {
-    for (int i = threadIdx.x; i < D; i += 64 * kMergeWaves) out[i] = 0;
-    // Fused append of a sequence with no keys to attend to: the first query
-    // head of each kv-head group writes that head's slice of the new row.
-    const int G = p.num_heads / p.num_kv_heads;
-    if (p.new_k != nullptr && h % G == 0) {
-      const int64_t slot = p.slot_mapping[b];
-      const int kh = h / G;
-      const int64_t row_stride = static_cast<int64_t>(p.num_kv_heads) * D;
-      const int64_t src = (static_cast<int64_t>(b) * p.num_kv_heads + kh) * D;
-      for (int i = threadIdx.x; slot >= 0 && i < D; i += 64 * kMergeWaves) {
-        const_cast<uint16_t*>(static_cast<const uint16_t*>(p.k))[slot * row_stride + kh * D + i] =
-            static_cast<const uint16_t*>(p.new_k)[src + i];
-        const_cast<uint16_t*>(static_cast<const uint16_t*>(p.v))[slot * row_stride + kh * D + i] =
-            static_cast<const uint16_t*>(p.new_v)[src + i];
-      }
-    }
+    empty_sequence<D>(p, b, h, 1, 64 * kMergeWaves);
     return;
   }
   const int lo = p.window_left >= 0 ? max(0, L - 1 - p.window_left) : 0;
@@ -1160,6 +1169,12 @@ int64_t choose_split_tokens(int64_t batch, int64_t num_kv_heads, int64_t max_seq
   // 256-key workgroups take 128-key splits: B=4 ctx 0.3k-1k 19.4 -> 16.9 us,
   // B=8 ctx 1-3000 18.4 -> 17.7 us (at 4096 workgroups, the 0.6B shape, the
   // longer merge outweighs the finer grid).
+  // Contexts of at most 256 keys take one split per sequence, which writes its output:
+  // no second launch.  Two launches -> one (256 keys by two splits before): 3 sequences
+  // of 20-100 keys 5.9 -> 4.6 us, of 20-250 7.9 -> 6.8, 16 of 100-256 (32 heads) 9.4 ->
+  // 7.7, 128 of 20-100 16.6 -> 13.2.  Few contexts of 512 keys would lose by it (one 8.2
+  // -> 9.8: the longer walk of one workgroup).
+  if (max_seqlen_k <= 256) return max_seqlen_k <= 128 ? 128 : 256;
   for (int64_t st : {int64_t{1024}, int64_t{512}}) {
     if (batch * num_kv_heads * ceil_div(max_seqlen_k, st) >= 4096) return st;
   }
@@ -1215,6 +1230,7 @@ bool dispatch_group(const DecodeParams& p, int64_t batch, int group, hipStream_t
 // splits) 12.8 -> 13.9, 4 of 4k-16k (128 splits, 128 pairs) 45.1 -> 46.2.
 template <class Tag, int D>
 void launch_split_merge(const DecodeParams& p, dim3 grid, hipStream_t s) {
+  if (p.max_splits == 1) return;  // pass 1 wrote every output
   if (p.max_splits >= 96 && p.num_heads * p.batch <= 64)
     hipLaunchKernelGGL((paged_decode_merge<Tag, D, 16, 16>), grid, dim3(1024), 0, s, p);
   else
