@@ -495,12 +495,13 @@ def test_decode_fused_append_equals_append_then_attend(device, case, decode_path
     assert np.array_equal(to_bits(v2), to_bits(v1))
 
 
-# Contexts of at most 128 / 256 keys: one split per sequence and no merge, empty
+# Contexts of at most 128 / 256 / 512 keys: one split per sequence and no merge, empty
 # sequences (their zeros and their append) included.
 SINGLE_SPLIT = [
     (5, 16, 8, 128, 256, 20, [0, 10, 0, 256, 129], -1, "bf16"),
     (4, 28, 4, 64, 16, 80, [128, 1, 0, 127], -1, "f16"),
     (3, 16, 2, 128, 32, 40, [250, 3, 0], 20, "bf16"),
+    (64, 8, 8, 64, 64, 320, [512, 0, 300, 129] * 16, -1, "bf16"),  # 512 workgroups: up to 512 keys
 ]
 
 

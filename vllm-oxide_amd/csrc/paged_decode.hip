@@ -1169,12 +1169,15 @@ int64_t choose_split_tokens(int64_t batch, int64_t num_kv_heads, int64_t max_seq
   // 256-key workgroups take 128-key splits: B=4 ctx 0.3k-1k 19.4 -> 16.9 us,
   // B=8 ctx 1-3000 18.4 -> 17.7 us (at 4096 workgroups, the 0.6B shape, the
   // longer merge outweighs the finer grid).
-  // Contexts of at most 256 keys take one split per sequence, which writes its output:
+  // Short contexts take one split per sequence, which writes its output:
   // no second launch.  Two launches -> one (256 keys by two splits before): 3 sequences
   // of 20-100 keys 5.9 -> 4.6 us, of 20-250 7.9 -> 6.8, 16 of 100-256 (32 heads) 9.4 ->
-  // 7.7, 128 of 20-100 16.6 -> 13.2.  Few contexts of 512 keys would lose by it (one 8.2
-  // -> 9.8: the longer walk of one workgroup).
+  // 7.7, 128 of 20-100 16.6 -> 13.2.  Contexts of up to 512 keys only from 512 workgroups
+  // on: 128 of 100-500 43.5 -> 38.9 us, but one of 500 8.2 -> 9.8 and 4 of 100-400 8.1 ->
+  // 10.1 (the longer walk of one workgroup); 64 of 200-1024 by one split of 1024 39.7 ->
+  // 39.2, left at 256.
   if (max_seqlen_k <= 256) return max_seqlen_k <= 128 ? 128 : 256;
+  if (max_seqlen_k <= 512 && batch * num_kv_heads >= 512) return 512;
   for (int64_t st : {int64_t{1024}, int64_t{512}}) {
     if (batch * num_kv_heads * ceil_div(max_seqlen_k, st) >= 4096) return st;
   }
