@@ -146,6 +146,27 @@ def test_prefill_many_prompts_vs_oracle(device, lens):
     assert_attn_close(got, oracle.prefill_attention(q, kc, vc, cuq, cuk, 0.125, table, -1, "bf16"))
 
 
+# (sequence, kv head) units that do not fill the 8 XCDs evenly: their row tiles alternate
+# over 8, 2 (12 units; tile counts 7 and 1), 4 and 8 (10 and 9 units) XCDs.
+UNEVEN = [
+    # (lq, Hq, Hkv, D, BS, window, dtype)
+    ([300], 8, 1, 128, 64, -1, "bf16"),
+    ([100, 1, 113], 28, 4, 128, 256, -1, "f16"),
+    ([70, 5, 64, 33, 129], 8, 2, 64, 16, 50, "bf16"),
+    ([40] * 9, 16, 1, 64, 256, -1, "bf16"),
+]
+
+
+@pytest.mark.parametrize("case", UNEVEN, ids=[f"u{i}" for i in range(len(UNEVEN))])
+def test_prefill_uneven_units_vs_oracle(device, case):
+    lens, Hq, Hkv, D, BS, window, dtype = case
+    q, kc, vc, cuq, cuk, table = _case(71, lens, lens, Hq, Hkv, D, BS, dtype)
+    scale = 1.0 / math.sqrt(D)
+    print(f"prefill uneven units lq={lens} Hq={Hq} Hkv={Hkv} D={D} BS={BS} w={window} {dtype}", flush=True)
+    got = to_f32(_gpu(device, q, kc, vc, cuq, cuk, table, scale, window, dtype))
+    assert_attn_close(got, oracle.prefill_attention(q, kc, vc, cuq, cuk, scale, table, window, dtype))
+
+
 # Queries behind long cached contexts, whose keys are split over workgroups: the piece
 # and tile edges, sequences with nothing to split or no queries, the smallest batch and
 # the largest that is split (64), rows of 128 that groups of 7 and 5 do not fill.

@@ -76,6 +76,8 @@ struct PrefillParams {
   int tokens_per_wg;
   int tiles_per_unit;
   int units;                   // batch * num_kv_heads
+  int spread;                  // XCDs that share a unit's row tiles (plain grid)
+  int share_tiles;             // row tiles of a unit per XCD of its share
   int block_size;
   int window_left;
   float scale_log2;
@@ -263,14 +265,17 @@ __global__ __launch_bounds__(kPfThreads, 2) void paged_prefill_attn(PrefillParam
   __shared__ __align__(1024) char smem1[BUF];
 
   // XCD-aware work item: unit (sequence, kv head) u sits on XCD u % 8 and its
-  // tiles are consecutive workgroups there, heaviest first.  Shared-prefix pass:
+  // tiles are consecutive workgroups there, heaviest first; where the units are no
+  // multiple of 8, each unit's tiles alternate over `spread` XCDs, so that all 8 get
+  // the same share.  Shared-prefix pass:
   // unit (key split, kv head), all of them over table row 0 (the shared entries).
   // Balanced launch: XCD x takes the x-th eighth of the pieces.
   const int i = blockIdx.x;
   const int j = i / kPfXcds;
-  const int u = (j / p.tiles_per_unit) * kPfXcds + i % kPfXcds;
-  if (!kSplit && u >= p.units) return;
-  const int jj = j % p.tiles_per_unit;
+  const int share = (j / p.share_tiles) * kPfXcds + i % kPfXcds;
+  const int u = share / p.spread;
+  const int jj = (j % p.share_tiles) * p.spread + share % p.spread;
+  if (!kSplit && (u >= p.units || jj >= p.tiles_per_unit)) return;
   // kPair: a workgroup takes row tiles n - 1 - jj and then jj (half of the workgroups
   // end at once) where the prompts are of about one length; in ragged batches the pairs
   // would be uneven.
@@ -864,8 +869,7 @@ bool launch_prefill(const PrefillParams& p, int head_dim, hipStream_t s) {
     head_dim == 128 ? launch_balanced<Tag, 128>(p, s) : launch_balanced<Tag, 64>(p, s);
     return true;
   }
-  const int64_t units8 = ceil_div64(p.units, kPfXcds) * kPfXcds;
-  const dim3 grid(static_cast<unsigned>(units8 * p.tiles_per_unit));
+  const dim3 grid(static_cast<unsigned>(ceil_div64(int64_t{p.units} * p.spread, kPfXcds) * kPfXcds * p.share_tiles));
   if (head_dim == 128) {
     launch_mode<Tag, 128>(p, grid, s);
     return true;
@@ -944,6 +948,15 @@ void prefill_impl(void* out, const void* q, const void* k, const void* v, const 
   }
   p.tiles_per_unit = static_cast<int>(tiles);
   p.units = static_cast<int>(units);
+  // Where whole units would load the 8 XCDs more than a fifth unevenly, a unit's tiles go
+  // to the fewest XCDs that make the shares a multiple of 8; otherwise its K/V stays in
+  // one L2.  One prompt of 4096 tokens on 28 heads / 4 kv heads 249 -> 131 us, on 8 heads
+  // / 1 kv head 204 -> 70, 3 of 2000 (12 units) 133 -> 115; 7 units of 3000 lose by it
+  // (148 -> 153).
+  p.spread = 1;
+  if (p.units < 1024 && 5 * ceil_div64(p.units, kPfXcds) * kPfXcds > 6 * int64_t{p.units})
+    while (p.units * p.spread % kPfXcds != 0) p.spread *= 2;
+  p.share_tiles = static_cast<int>(ceil_div64(tiles, p.spread));
   // Prompts with no cached prefix, of at most 2048 tokens and about one length (the
   // kernel looks), with work for four rounds of the chip's slots: a workgroup takes a
   // unit's row tiles n - 1 - i and then i (a separate kernel instance), the same keys per
@@ -951,7 +964,7 @@ void prefill_impl(void* out, const void* q, const void* k, const void* v, const 
   // 62.7 us, 16 x 1024 188 -> 184, 8 x 2048 303 -> 296; smaller or ragged batches lose
   // (1 x 300 11.6 -> 17.0, 128 x 128 51 -> 62, 8 of 200-1000 81 -> 89), and so do 4 x
   // 4096 and prompts behind a cached prefix, whose tiles already carry equal keys.
-  p.pair = (tiles >= 8 && max_seqlen_k <= max_seqlen_q && max_seqlen_q <= 2048 &&
+  p.pair = (tiles >= 8 && p.spread == 1 && max_seqlen_k <= max_seqlen_q && max_seqlen_q <= 2048 &&
             tiles * units >= 8 * static_cast<int64_t>(oxide::device_cu_count()))
                ? 1
                : 0;
@@ -1062,6 +1075,8 @@ bool launch_decode_prefix(const DecodePrefixArgs& a, hipStream_t s) {
   p.tokens_per_wg = kPfRows / p.group;
   p.tiles_per_unit = static_cast<int>(ceil_div64(a.batch, p.tokens_per_wg));
   p.units = a.num_kv_heads * a.pre_splits;
+  p.spread = 1;
+  p.share_tiles = p.tiles_per_unit;
   p.block_size = a.block_size;
   p.window_left = a.window_left < 0 ? -1 : a.window_left;
   p.scale_log2 = a.scale_log2;
