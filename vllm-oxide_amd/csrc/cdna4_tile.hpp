@@ -80,9 +80,7 @@ __device__ __forceinline__ uint2 lds_read_tr16(const char* p) {
 }
 
 // Two fp32 values -> packed 16-bit pair of the MFMA input type, round to
-// nearest even, one instruction: v_cvt_pk_bf16_f32, v_cvt_pk_f16_f32 (as two
-// conversions and an or: 32 more VALU operations per 64-key step of f16 prefill, 4 x 4096
-// 561 -> 574 us, 8 x 2048 at D = 64 176 -> 185).
+// nearest even (bf16: one v_cvt_pk_bf16_f32).
 typedef float float2_t __attribute__((ext_vector_type(2)));
 typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
 typedef _Float16 f16x2_t __attribute__((ext_vector_type(2)));
@@ -90,6 +88,15 @@ __device__ __forceinline__ uint32_t pack2(Bf16Tag, float lo, float hi) {
   return __builtin_bit_cast(uint32_t, __builtin_convertvector((float2_t){lo, hi}, bf16x2_t));
 }
 __device__ __forceinline__ uint32_t pack2(F16Tag, float lo, float hi) {
+  return static_cast<uint32_t>(pack1(F16Tag{}, lo)) | (static_cast<uint32_t>(pack1(F16Tag{}, hi)) << 16);
+}
+// The same with one conversion for f16 too (v_cvt_pk_f16_f32).  pack2's two and an or
+// are 32 more VALU operations per 64-key step of f16 prefill (4 x 4096 574 -> 561 us, 8
+// x 2048 at D = 64 185 -> 176); where the values are products, pack2 lets each multiply
+// and conversion fuse (decode: 0.5 % faster so), and the prologue's f16 instances would
+// spill with this form.
+__device__ __forceinline__ uint32_t pack2_cvt(Bf16Tag, float lo, float hi) { return pack2(Bf16Tag{}, lo, hi); }
+__device__ __forceinline__ uint32_t pack2_cvt(F16Tag, float lo, float hi) {
   return __builtin_bit_cast(uint32_t, __builtin_convertvector((float2_t){lo, hi}, f16x2_t));
 }
 

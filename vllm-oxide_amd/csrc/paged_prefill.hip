@@ -606,10 +606,10 @@ __global__ __launch_bounds__(kPfThreads, 2) void paged_prefill_attn(PrefillParam
         for (int r = 0; r < 16; ++r) x[r] = __builtin_amdgcn_exp2f(__builtin_fmaf(sc[kb][r], c_log2, -msafe));
 #pragma unroll
         for (int s2 = 0; s2 < 2; ++s2) {
-          pb[kb][s2].x = pack2(Tag{}, x[8 * s2 + 0], x[8 * s2 + 1]);
-          pb[kb][s2].y = pack2(Tag{}, x[8 * s2 + 2], x[8 * s2 + 3]);
-          pb[kb][s2].z = pack2(Tag{}, x[8 * s2 + 4], x[8 * s2 + 5]);
-          pb[kb][s2].w = pack2(Tag{}, x[8 * s2 + 6], x[8 * s2 + 7]);
+          pb[kb][s2].x = pack2_cvt(Tag{}, x[8 * s2 + 0], x[8 * s2 + 1]);
+          pb[kb][s2].y = pack2_cvt(Tag{}, x[8 * s2 + 2], x[8 * s2 + 3]);
+          pb[kb][s2].z = pack2_cvt(Tag{}, x[8 * s2 + 4], x[8 * s2 + 5]);
+          pb[kb][s2].w = pack2_cvt(Tag{}, x[8 * s2 + 6], x[8 * s2 + 7]);
           lsum = sum2_acc(Tag{}, pb[kb][s2].x, lsum);
           lsum = sum2_acc(Tag{}, pb[kb][s2].y, lsum);
           lsum = sum2_acc(Tag{}, pb[kb][s2].z, lsum);
@@ -709,8 +709,8 @@ __global__ __launch_bounds__(kPfThreads, 2) void paged_prefill_attn(PrefillParam
 #pragma unroll
       for (int q = 0; q < 4; ++q) {
         uint2 w;
-        w.x = pack2(Tag{}, acc[db][4 * q + 0] * inv, acc[db][4 * q + 1] * inv);
-        w.y = pack2(Tag{}, acc[db][4 * q + 2] * inv, acc[db][4 * q + 3] * inv);
+        w.x = pack2_cvt(Tag{}, acc[db][4 * q + 0] * inv, acc[db][4 * q + 1] * inv);
+        w.y = pack2_cvt(Tag{}, acc[db][4 * q + 2] * inv, acc[db][4 * q + 3] * inv);
         *reinterpret_cast<uint2*>(op + 32 * db + 8 * q) = w;
       }
   }
@@ -776,8 +776,8 @@ __global__ __launch_bounds__(256) void paged_prefill_merge(PrefillParams p) {
     }
     const float inv = l > 0.f ? 1.f / l : 0.f;
     uint2 out;
-    out.x = pack2(Tag{}, o.x * inv, o.y * inv);
-    out.y = pack2(Tag{}, o.z * inv, o.w * inv);
+    out.x = pack2_cvt(Tag{}, o.x * inv, o.y * inv);
+    out.y = pack2_cvt(Tag{}, o.z * inv, o.w * inv);
     *reinterpret_cast<uint2*>(static_cast<uint16_t*>(p.out) + ((q0 + tq) * p.num_heads + kh * G + r % G) * D + 4 * c) =
         out;
   }

@@ -37,14 +37,6 @@
 
 namespace {
 
-// Two fp32 values -> a packed 16-bit pair.  f16 converts them one by one: with
-// v_cvt_pk_f16_f32 (pack2) the kernel's f16 instances spill 8 registers at their 96.
-__device__ __forceinline__ uint32_t pack_pair(Bf16Tag, float lo, float hi) { return pack2(Bf16Tag{}, lo, hi); }
-__device__ __forceinline__ uint32_t pack_pair(F16Tag, float lo, float hi) {
-  return static_cast<uint32_t>(pack1(F16Tag{}, lo)) | (static_cast<uint32_t>(pack1(F16Tag{}, hi)) << 16);
-}
-
-
 constexpr int kRopeThreads = 256;
 template <int D>
 constexpr int kLanesPerHead = D / 16;  // 8 elements of each half per lane
@@ -72,7 +64,7 @@ __device__ __forceinline__ float weigh(float x, float w) {
 // and widen it back: the reference's "to dtype" steps between fp32 operations.
 template <class Tag>
 __device__ __forceinline__ void round_pair(float& a, float& b) {
-  const uint32_t u = pack_pair(Tag{}, a, b);
+  const uint32_t u = pack2(Tag{}, a, b);
   a = to_f32(Tag{}, static_cast<uint16_t>(u));
   b = to_f32(Tag{}, static_cast<uint16_t>(u >> 16));
 }
@@ -292,8 +284,8 @@ __device__ __forceinline__ void rope_task(const RopeParams& p, const TaskIn& in,
   uint32_t y1[E / 2], y2[E / 2];  // packed pairs
 #pragma unroll
   for (int e = 0; e < E; e += 2) {
-    y1[e / 2] = pack_pair(Tag{}, x1[e] * sd.c[e] - x2[e] * sd.s[e], x1[e + 1] * sd.c[e + 1] - x2[e + 1] * sd.s[e + 1]);
-    y2[e / 2] = pack_pair(Tag{}, x2[e] * sd.c[e] + x1[e] * sd.s[e], x2[e + 1] * sd.c[e + 1] + x1[e + 1] * sd.s[e + 1]);
+    y1[e / 2] = pack2(Tag{}, x1[e] * sd.c[e] - x2[e] * sd.s[e], x1[e + 1] * sd.c[e + 1] - x2[e + 1] * sd.s[e + 1]);
+    y2[e / 2] = pack2(Tag{}, x2[e] * sd.c[e] + x1[e] * sd.s[e], x2[e + 1] * sd.c[e + 1] + x1[e + 1] * sd.s[e + 1]);
   }
   uint16_t* dst0;
   uint16_t* dst1 = nullptr;
