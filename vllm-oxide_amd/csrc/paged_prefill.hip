@@ -401,14 +401,14 @@ __global__ __launch_bounds__(kPfThreads, 2) void paged_prefill_attn(PrefillParam
   const uint32_t strideb = static_cast<uint32_t>(row_stride * 2);
   int trow[NLD];
   uint32_t rowb[NLD], kchb[NLD], vchb[NLD];
-  int blk_row[NLD];  // kPagedRows: the next tile's block ids
+  int blk_row[NLD], in_row[NLD];  // kPagedRows: the next tile's block ids, the rows inside them
 #pragma unroll
   for (int x = 0; x < NLD; ++x) {
     trow[x] = wave * WROWS + x * RPI + lrow;
     kchb[x] = 16 * (lpos ^ kswz<D>(trow[x]));
     vchb[x] = 32 * ((lpos >> 1) ^ vswz<D>(trow[x])) + 16 * (lpos & 1);
     rowb[x] = static_cast<uint32_t>(trow[x]) * strideb;
-    blk_row[x] = 0;
+    blk_row[x] = in_row[x] = 0;
   }
   // The tile being fetched (tiles are fetched in order): its first key, and for
   // kPagedTiles its page, the offset inside it, that page's block and the next one's.
@@ -422,10 +422,18 @@ __global__ __launch_bounds__(kPfThreads, 2) void paged_prefill_attn(PrefillParam
     f_next = bt[min(f_page + 1, last_page)];
   }
   // kPagedRows: block ids of the tile at f_kb, read a tile ahead of its loads.
+  // One division per row and tile: taking the remainder again at each of the row's loads
+  // cost 64 more VALU operations between a step's score MFMAs (pages of 16, 4 x 2048
+  // 169 -> 180 us).
   auto fetch_rows = [&]() {
     if (MODE == kPagedRows) {
 #pragma unroll
-      for (int x = 0; x < NLD; ++x) blk_row[x] = p.block_table[b * p.max_blocks + min(f_kb + trow[x], Lk - 1) / p.block_size];
+      for (int x = 0; x < NLD; ++x) {
+        const uint32_t key = min(f_kb + trow[x], Lk - 1);
+        const uint32_t entry = key / static_cast<uint32_t>(p.block_size);
+        blk_row[x] = p.block_table[b * p.max_blocks + entry];
+        in_row[x] = static_cast<int>(key - entry * p.block_size);
+      }
     }
   };
   // Wave-uniform source of the tile at f_kb: base rows and the byte offset of its
@@ -454,9 +462,8 @@ __global__ __launch_bounds__(kPfThreads, 2) void paged_prefill_attn(PrefillParam
     const uint32_t dst = sbuf + (wave * WROWS + x * RPI) * ROWB + (x2 & 1) * TBYTES;
     if (MODE == kPagedRows) {
       // General pages: a 64-bit source address per lane.
-      const int key = min(f_kb + trow[x], Lk - 1);
       const int blk = min(max(blk_row[x], 0), p.num_blocks - 1);
-      const int64_t row = static_cast<int64_t>(blk) * p.block_size + key % p.block_size;
+      const int64_t row = static_cast<int64_t>(blk) * p.block_size + in_row[x];
       if (x2 & 1)
         load_lds16(vbase + row * row_stride + vchb[x] / 2, dst);
       else
