@@ -5,7 +5,7 @@ cmake, no JIT cache), so the .so travels with the source tree.  Every call
 recompiles.  Counterpart of the reference's crates/vllm-oxide/build.rs:1-30
 (nvcc via cudaforge -> static lib); here hipcc --offload-arch=gfx950 -> the
 shared library Python loads with ctypes, plus the same objects archived as
-liboxide_paged_kv.a.  rust/oxide-paged-kv-sys/build.rs and
+liboxide_paged_kv.a, and the Python ops' native module against torch's headers.  rust/oxide-paged-kv-sys/build.rs and
 vllm-oxide_amd/Makefile compile the same sources with the same flags.
 """
 from __future__ import annotations

@@ -92,9 +92,9 @@ __device__ __forceinline__ uint32_t pack2(F16Tag, float lo, float hi) {
 }
 // The same with one conversion for f16 too (v_cvt_pk_f16_f32).  pack2's two and an or
 // are 32 more VALU operations per 64-key step of f16 prefill (4 x 4096 574 -> 561 us, 8
-// x 2048 at D = 64 185 -> 176); where the values are products, pack2 lets each multiply
-// and conversion fuse (decode: 0.5 % faster so), and the prologue's f16 instances would
-// spill with this form.
+// x 2048 at D = 64 185 -> 176).  Decode keeps pack2: its values are products, whose
+// multiply and conversion fuse into one rounding there (35.9 us either way for 23
+// sequences on 40 heads); the prologue's f16 instances would spill with this form.
 __device__ __forceinline__ uint32_t pack2_cvt(Bf16Tag, float lo, float hi) { return pack2(Bf16Tag{}, lo, hi); }
 __device__ __forceinline__ uint32_t pack2_cvt(F16Tag, float lo, float hi) {
   return __builtin_bit_cast(uint32_t, __builtin_convertvector((float2_t){lo, hi}, f16x2_t));

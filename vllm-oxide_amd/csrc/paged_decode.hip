@@ -45,7 +45,7 @@
 // With the fused append (paged_decode_attention_append) the workgroup whose
 // keys include position L-1 first writes its kv head's slice of the new
 // token's K/V to slot_mapping[b] and uses those values for that key.
-// Pass 2 (paged_decode_merge): 4 waves per (query head, sequence) merge the
+// Pass 2 (paged_decode_merge): 4 or 16 waves per (query head, sequence) merge the
 // splits that intersect [lo, L) with log-sum-exp weights and write out.
 //
 // Every path reads K/V exactly once; the partials add 2 * Hq * (D+1) * 4 bytes

@@ -1,8 +1,8 @@
 """MI355X (gfx950) paged-KV hot path of vllm-oxide: Python front end.
 
 The kernels live in liboxide_paged_kv.so (HIP, built in-tree by
-vllm-oxide_amd/build.py); this package only binds them (ctypes) and generates
-the synthetic workloads of the benchmark configurations.
+vllm-oxide_amd/build.py); this package binds them (ctypes, and _native.so for the
+calls of a serving step) and generates the synthetic workloads of the benchmark configurations.
 """
 from ._lib import LIB_PATH, OxideError, load  # noqa: F401
 from .ops import (CASCADE_MODES, DECODE_PATHS, build_decode_metadata, copy_blocks, decode_attn,  # noqa: F401
