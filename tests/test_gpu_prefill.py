@@ -278,3 +278,30 @@ def test_prefill_last_rows_equal_decode(device, window):
                          torch.from_numpy(table).to(device), max(lk), 0.09, None if window < 0 else window)
     torch.cuda.synchronize()
     assert_attn_close(pre[last], to_f32(dec))
+
+
+# An infinite or NaN V reaches only rows whose wave (32 rows) sees some key of its 64-key
+# tile.  Group 1: a wave is 32 tokens, a workgroup 128.  (window, cached, bad key, the
+# tokens of waves that see nothing of the key's tile)
+BAD_V = [
+    (-1, 0, 200, (0, 192)),      # keys of tile 192..255 are after every token below 192
+    (20, 0, 70, (160, 256)),     # window 20: tokens from 160 on see keys from 140 on
+    (-1, 4096, 200, (0, 192)),   # the same behind a cached context, keys split over workgroups
+    (20, 4096, 70, (160, 256)),
+]
+
+
+@pytest.mark.parametrize("case", BAD_V, ids=["causal", "window", "causal-cached", "window-cached"])
+@pytest.mark.parametrize("BS", [64, 16])
+@pytest.mark.parametrize("bad", [np.nan, np.inf])
+def test_prefill_bad_values_stay_in_their_tile(device, case, BS, bad):
+    window, cached, key, (lo, hi) = case
+    q, kc, vc, cuq, cuk, table = _case(81, [256], [256 + cached], 1, 1, 64, BS)
+    print(f"prefill bad V window={window} cached={cached} BS={BS} {bad}", flush=True)
+    clean = to_f32(_gpu(device, q, kc, vc, cuq, cuk, table, 0.125, window, "bf16"))
+    vb = vc.copy()
+    j = cached + key
+    vb[table[0, j // BS], j % BS] = oracle.f32_to_bf16_bits(np.full((1, 64), bad, np.float32))
+    got = to_f32(_gpu(device, q, kc, vb, cuq, cuk, table, 0.125, window, "bf16"))
+    assert not np.isfinite(got[key]).any()  # the token itself sees the key
+    assert np.array_equal(got[lo:hi], clean[lo:hi])

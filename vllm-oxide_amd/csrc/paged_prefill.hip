@@ -374,9 +374,18 @@ __global__ __launch_bounds__(kPfThreads, 2) void paged_prefill_attn(PrefillParam
     hi_r = valid ? khi : -1;
     lo_r = valid && W >= 0 ? L - 1 - W : 0;
   }
-  // Whether the wave has rows at all.
+  // The wave's own tiles [it0, it1): those in which some row of it sees a key (none
+  // without rows).  The others it only loads for the rest.
   const int wr0 = wave * 32;
-  const bool wave_active = wr0 < rows_used && t0 + wr0 / G < t1;
+  const int wt_first = t0 + wr0 / G;
+  int it0 = ntiles, it1 = ntiles;
+  if (wr0 < rows_used && wt_first < t1) {
+    const int wt_last = min(t1 - 1, t0 + min(wr0 + 31, rows_used - 1) / G);
+    const int wave_hi = kPrefix ? khi : min(Lk - 1, wt_last + off);
+    const int wave_lo = !kPrefix && W >= 0 ? wt_first + off - W : 0;
+    it1 = wave_hi >= kt0 ? min(ntiles, (wave_hi - kt0) / kPfKeys + 1) : 0;
+    it0 = wave_lo > kt0 ? min(it1, (wave_lo - kt0) / kPfKeys) : 0;
+  }
 
   // Queries (B operand of S^T, 16 dims per k-step).  A negative scale is
   // applied as a sign flip of q (exact) and |scale|, so the running maxima can
@@ -669,22 +678,29 @@ __global__ __launch_bounds__(kPfThreads, 2) void paged_prefill_attn(PrefillParam
     }
   }
 
-  if (wave_active) {
-    for (int it = 0; it < ntiles; it += 2) {
-      step(it, smem0, lds1);
-      if (it + 1 < ntiles) step(it + 1, smem1, lds0);
-    }
-  } else {
-    // A wave without rows only loads its share of the tiles (a branch around the math
-    // inside step would cost every wave copies of its accumulators where it joins).
-    for (int it = 0; it < ntiles; ++it) {
+  // A tile that no row of the wave sees is left out of its math: P is 0 there, but 0
+  // times an infinite or NaN V is not.  The loops are split at the borders because a
+  // branch around the math inside step would cost every wave copies of its accumulators
+  // where it joins.  Against running every tile of the workgroup, one query head per kv
+  // head: 16 x 1024 115 -> 109 us, with a window of 128 66 -> 63; 4 x 2048, and groups of
+  // two and four with or without a window, within 1 %.
+  auto load_only = [&](int from, int to) {
+    for (int it = from; it < to; ++it) {
       asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
       __syncthreads();
 #pragma unroll
       for (int x = 0; x < 2 * NLD; ++x) issue_load(x, it % 2 == 0 ? lds1 : lds0);
       next_tile();
     }
+  };
+  load_only(0, it0);
+  int it = it0;
+  if (it0 % 2 == 1 && it0 < it1) step(it++, smem1, lds0);
+  for (; it < it1; it += 2) {
+    step(it, smem0, lds1);
+    if (it + 1 < it1) step(it + 1, smem1, lds0);
   }
+  load_only(it1, ntiles);
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the last step's loads, before the wave ends
 
   // out[row][d] for d = 32 db + 8 q + 4 half + e (register 4 q + e), normalised
