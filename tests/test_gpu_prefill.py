@@ -305,3 +305,64 @@ def test_prefill_bad_values_stay_in_their_tile(device, case, BS, bad):
     got = to_f32(_gpu(device, q, kc, vb, cuq, cuk, table, 0.125, window, "bf16"))
     assert not np.isfinite(got[key]).any()  # the token itself sees the key
     assert np.array_equal(got[lo:hi], clean[lo:hi])
+
+
+def _entry(device, q, k, v, cuq, cuk, table, scale, window, dtype, workspace_bytes=None, offset=0):
+    """The C entries: paged_prefill_attention, or with workspace_bytes the workspace form
+    over that many bytes from `offset` of a guarded buffer (0 = no workspace).  Returns
+    the output and whether the bytes outside the stated workspace are as they were."""
+    import torch
+    from oxide_paged_kv import _lib
+
+    L = _lib.load()
+    t = lambda a: to_torch(a, dtype, device)  # noqa: E731
+    i32 = lambda a: torch.from_numpy(a.view(np.int32)).to(device)  # noqa: E731
+    qd, kd, vd, cq, ck, tb = t(q), t(k), t(v), i32(cuq), i32(cuk), i32(table)
+    out = torch.zeros_like(qd)
+    (_, Hq, D), (NB, BS, Hkv, _) = q.shape, k.shape
+    args = [out, qd, kd, vd, cq, ck, tb]
+    sizes = [table.shape[1], NB, len(cuq) - 1, Hq, Hkv, D, BS, int(np.max(np.diff(cuq))), int(np.max(np.diff(cuk))),
+             window, scale]
+    code, stream = _lib.DTYPE_BF16 if dtype == "bf16" else _lib.DTYPE_F16, torch.cuda.current_stream().cuda_stream
+    guard = torch.full(((workspace_bytes or 0) + 8192,), 0x5A, dtype=torch.uint8, device=device)
+    ptrs = [a.data_ptr() for a in args]
+    if workspace_bytes is None:
+        L.paged_prefill_attention(*ptrs, *sizes, code, stream)
+    else:
+        L.paged_prefill_attention_workspace(*ptrs, *sizes, guard.data_ptr() + offset if workspace_bytes else None,
+                                            workspace_bytes, code, stream)
+    _lib.check()
+    torch.cuda.synchronize()
+    return out, bool((guard[:offset] == 0x5A).all()) and bool((guard[offset + (workspace_bytes or 0):] == 0x5A).all())
+
+
+def _workspace_size(q, k, cuq, cuk, window):
+    from oxide_paged_kv import _lib
+
+    return int(_lib.load().prefill_attention_workspace_size(
+        len(cuq) - 1, q.shape[1], k.shape[2], q.shape[2], int(np.max(np.diff(cuq))), int(np.max(np.diff(cuk))), window))
+
+
+@pytest.mark.parametrize("lk", [1500, 2600])  # three and six pieces of a row tile
+@pytest.mark.parametrize("what", ["q nan", "q inf", "k nan", "v inf last", "v inf first", "v nan"])
+def test_prefill_split_keys_pass_nan_and_infinity(device, lk, what):
+    """NaN and infinities come out of keys split over workgroups as from the plain entry."""
+    q, kc, vc, cuq, cuk, table = _case(83, [3], [lk], 8, 2, 64, 64)
+    bits = lambda x: oracle.f32_to_bf16_bits(np.full((), x, np.float32))  # noqa: E731
+    at = lambda j: (table[0, j // 64], j % 64)  # noqa: E731
+    if what[0] == "q":
+        q[1] = bits(np.nan if "nan" in what else np.inf)
+    elif what[0] == "k":
+        kc[at(700)] = bits(np.nan)
+    else:
+        vc[at(3 if "first" in what else lk - 10)] = bits(np.nan if "nan" in what else np.inf)
+    need = _workspace_size(q, kc, cuq, cuk, -1)
+    assert need > 0
+    print(f"prefill split lk={lk} {what}", flush=True)
+    want = to_f32(_entry(device, q, kc, vc, cuq, cuk, table, 0.125, -1, "bf16")[0])
+    got = to_f32(_entry(device, q, kc, vc, cuq, cuk, table, 0.125, -1, "bf16", need)[0])
+    assert not np.isfinite(want).all()
+    assert np.array_equal(np.isnan(got), np.isnan(want)) and np.array_equal(np.isinf(got), np.isinf(want))
+    fin = np.isfinite(want)
+    assert np.array_equal(np.sign(got[np.isinf(want)]), np.sign(want[np.isinf(want)]))
+    assert_attn_close(got[fin], want[fin])

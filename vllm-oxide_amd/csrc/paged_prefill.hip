@@ -722,7 +722,9 @@ __global__ __launch_bounds__(kPfThreads, 2) void paged_prefill_attn(PrefillParam
         *reinterpret_cast<float4*>(po + 32 * db + 8 * q) =
             make_float4(acc[db][4 * q + 0] * inv, acc[db][4 * q + 1] * inv, acc[db][4 * q + 2] * inv,
                         acc[db][4 * q + 3] * inv);
-    if (half == 0) p.part_lse[prow] = l > 0.f ? m_r + log2f(l) : -INFINITY;
+    // A row whose sum is NaN says so in kSplit, whose merge would take -inf for no keys.
+    const bool sums = kSplit ? l != 0.f : l > 0.f;
+    if (half == 0) p.part_lse[prow] = sums ? m_r + log2f(l) : -INFINITY;
   } else if (valid) {
     const float l = lsum;
     const float inv = l > 0.f ? 1.f / l : 0.f;
@@ -779,7 +781,11 @@ __global__ __launch_bounds__(256) void paged_prefill_merge(PrefillParams p) {
 #pragma unroll
       for (int z = 0; z < 4; ++z) v[z] = *reinterpret_cast<const float4*>(p.part_o + row(y + z) * D + 4 * c);
       const float mn = fmaxf(fmaxf(m, fmaxf(e[0], e[1])), fmaxf(e[2], e[3]));
-      if (mn == -INFINITY) continue;
+      // fmaxf passes NaN over: only pieces without keys may be left out.
+      if (mn == -INFINITY && e[0] == mn && e[1] == mn && e[2] == mn && e[3] == mn) continue;
+#pragma unroll
+      for (int z = 1; z < 4; ++z)  // past the last piece: its row again, maybe infinite
+        if (y + z >= n) v[z] = make_float4(0.f, 0.f, 0.f, 0.f);
       const float a = __builtin_amdgcn_exp2f(m - mn);
       m = mn;
       l *= a;
