@@ -327,8 +327,9 @@ void paged_prefill_attention(void* out, const void* q, const void* k_cache, cons
  * the chip idle or end unevenly, their keys are split over equal workgroups, whose
  * fp32 partial rows (in the workspace, no initialisation needed) a second kernel joins
  * by their log-sum-exps.  No reference counterpart.  Same results within rounding;
- * where splitting does not pay, or with a workspace that is NULL, not 16-byte aligned
- * or smaller than prefill_attention_workspace_size(...), it is
+ * where splitting does not pay (the kernel looks at the sequences' real lengths), or
+ * with a workspace that is NULL, not 16-byte aligned or smaller than
+ * prefill_attention_workspace_size(...), the results are those of
  * paged_prefill_attention itself.  Calls that share a workspace must not overlap in
  * time.
  */

@@ -366,3 +366,37 @@ def test_prefill_split_keys_pass_nan_and_infinity(device, lk, what):
     fin = np.isfinite(want)
     assert np.array_equal(np.sign(got[np.isinf(want)]), np.sign(want[np.isinf(want)]))
     assert_attn_close(got[fin], want[fin])
+
+
+# The balanced launch on the real lengths: (lq, lk, whether tiles are cut).  16 query heads
+# on one kv head (8 tokens per row tile), 256 CUs with two slots each.
+REAL_LENGTHS = [
+    ([256] * 8, [4096] * 8, False),                               # 256 tiles of one length
+    ([128] * 28, [7600 + 21 * i for i in range(28)], False),      # 448 tiles of about one length
+    ([128] * 40, [3328 + 28 * i for i in range(40)], False),      # 640 tiles: more than slots
+    ([256] * 8, [1024 + 438 * i for i in range(8)], True),        # 256 ragged ones
+    ([128] * 40, [500] * 39 + [12000], True),                     # 640, one sequence far longer
+    ([1024], [8704], True),                                       # pieces in one round
+    ([704, 1024], [4096, 6144], True),                            # and in two
+]
+
+
+@pytest.mark.parametrize("case", REAL_LENGTHS, ids=[f"r{i}" for i in range(len(REAL_LENGTHS))])
+def test_prefill_cuts_tiles_where_the_lengths_call_for_it(device, case):
+    """Where whole tiles take no longer the workspace entry is the plain one, bit for bit;
+    elsewhere it differs by rounding only."""
+    import torch
+
+    lq, lk, cut = case
+    if torch.cuda.get_device_properties(device).multi_processor_count != 256:
+        pytest.skip("the sizes are for 256 CUs")
+    q, kc, vc, cuq, cuk, table = _case(85, lq, lk, 16, 1, 128, 256)
+    need = _workspace_size(q, kc, cuq, cuk, -1)
+    assert need > 0
+    print(f"prefill real lengths lq={lq[:2]} lk={lk[:2]}", flush=True)
+    want, _ = _entry(device, q, kc, vc, cuq, cuk, table, 0.09, -1, "bf16")
+    got, _ = _entry(device, q, kc, vc, cuq, cuk, table, 0.09, -1, "bf16", need)
+    again, _ = _entry(device, q, kc, vc, cuq, cuk, table, 0.09, -1, "bf16", need)
+    assert torch.equal(got, again)
+    assert torch.equal(got, want) != cut
+    assert_attn_close(to_f32(got), to_f32(want))

@@ -101,6 +101,7 @@ struct PrefillParams {
   // batch size.  Partial rows go to part_o / part_lse, row piece * kPfRows + row.
   int max_pieces;
   int slots;       // workgroups that run at once
+  int may_be_whole;  // whether it asks the real lengths if cutting pays
   int batch;
   int* piece_len;  // the piece length chosen (workgroup 0 writes it, the merge reads it)
 };
@@ -117,7 +118,9 @@ __device__ __forceinline__ int clamp_len(int64_t n, int cap) {
 // workgroup then streams its own keys: 337 us for two chunks behind 16k-24k keys
 // against 300-310 with the pieces.)  The piece length is the shortest for which all
 // pieces run at once (slots workgroups), or in two rounds where rounding to whole
-// pieces costs the single round more than an eighth.
+// pieces costs the single round more than an eighth; where the lengths are such that
+// whole tiles take no longer (plain_us, split_us), no tile is cut and the merge ends at
+// once.
 // Lane b of every wave holds sequence b's entry (so at most 64 sequences).
 constexpr int kPfSplitBatch = 64;
 constexpr int kPfMinPiece = 8;
@@ -128,6 +131,7 @@ struct SeqPieces {
   int n;       // pieces of a tile
   int first;   // number of its first piece
   int total;   // all sequences' pieces (the same in every lane)
+  bool whole;  // no tile is cut (the same in every lane)
 };
 __host__ __device__ __forceinline__ int steps_per_tile(int keys, int window_left, int tokens_per_wg) {
   const int all = (keys + kPfKeys - 1) / kPfKeys;
@@ -146,13 +150,43 @@ __device__ __forceinline__ int wave_scan(int v) {
   return v;
 }
 __device__ __forceinline__ int wave_total(int v) { return __builtin_amdgcn_readlane(wave_scan(v), 63); }
+// The largest of the lanes' non-negative values.
+__device__ __forceinline__ int wave_max(int v) {
+  v = max(v, __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, false));
+  v = max(v, __builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, false));
+  v = max(v, __builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, false));
+  v = max(v, __builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, false));
+  v = max(v, __builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, false));
+  v = max(v, __builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false));
+  return __builtin_amdgcn_readlane(v, 63);
+}
+
+// Expected times, in us, of whole tiles in the plain order (work steps in all, the longest
+// tile's longest) and of pieces of at most len steps, start-up aside.  A step (128 rows x
+// 64 keys) takes about 1.06 us with one workgroup on a CU and 1.9 with two at D = 128,
+// 0.75 and 1.1 at D = 64.  More tiles than slots end raggedly: 640 tiles of 128 steps 380
+// us, of 98-125 335 whole and 417 cut.
+__host__ __device__ __forceinline__ float plain_us(int tiles, int work, int longest, int slots, int d) {
+  const float alone = d == 128 ? 1.06f : 0.75f, both = d == 128 ? 1.9f : 1.1f;
+  if (2 * tiles <= slots) return alone * longest;
+  const float once = alone * longest + (both - alone) * (static_cast<float>(work) / tiles);
+  return tiles > slots ? fmaxf(once, 1.25f * both * work / slots) : once;
+}
+// Each piece writes and the merge reads fp32 rows; the merge is a launch, and a piece
+// starts up as a tile does.
+__host__ __device__ __forceinline__ float split_us(int pieces, int tiles, int work, int len, int slots, int d) {
+  const float alone = d == 128 ? 1.06f : 0.75f, both = d == 128 ? 1.9f : 1.1f;
+  const float steps = 2 * pieces <= slots ? alone * len
+                      : pieces <= slots   ? both * len
+                                          : both * (tiles > slots ? 1.6f : 1.15f) * work / slots;
+  return steps + 1e-4f * d * pieces + 7.f;
+}
+constexpr int kPfWhole = INT32_MAX;  // the piece length stored where no tile is cut
 
 // The shortest piece length, at least kPfMinPiece, at which the sequences (units row
-// tiles of steps steps each, per lane) make at most `slots` pieces.
-__device__ __forceinline__ int shortest_piece(int units, int steps, int slots) {
+// tiles of steps steps each, per lane; tiles and work in all) make at most `slots` pieces.
+__device__ __forceinline__ int shortest_piece(int units, int steps, int slots, int tiles, int work) {
   // units * steps / len <= pieces <= units * (steps / len + 1) bound the bisection.
-  const int tiles = wave_total(units);
-  const int work = wave_total(units * steps);
   int lo = max(kPfMinPiece, (work + slots - 1) / slots);
   int hi = slots > tiles ? max(lo, (work + slots - tiles - 1) / (slots - tiles)) : INT32_MAX / 2;
   while (lo < hi) {
@@ -165,7 +199,7 @@ __device__ __forceinline__ int shortest_piece(int units, int steps, int slots) {
   return lo;
 }
 // kMerge: the piece length comes from the first pass.
-template <bool kMerge>
+template <bool kMerge, int D>
 __device__ __forceinline__ SeqPieces seq_pieces(const PrefillParams& p) {
   const int lane = threadIdx.x & 63;
   SeqPieces s{};
@@ -181,14 +215,23 @@ __device__ __forceinline__ SeqPieces seq_pieces(const PrefillParams& p) {
   if (kMerge) {
     len = __builtin_amdgcn_readfirstlane(*p.piece_len);
   } else {
-    len = shortest_piece(units, s.steps, p.max_pieces);
-    if (p.max_pieces > p.slots && wave_total(units) <= p.slots) {
-      const int one = shortest_piece(units, s.steps, p.slots);
+    const int tiles = wave_total(units), work = wave_total(units * s.steps);
+    len = shortest_piece(units, s.steps, p.max_pieces, tiles, work);
+    if (p.max_pieces > p.slots && tiles <= p.slots) {
+      const int one = shortest_piece(units, s.steps, p.slots, tiles, work);
       if (8 * one <= 18 * len) len = one;
+    }
+    if (p.may_be_whole) {
+      const int longest = wave_max(units > 0 ? s.steps : 0);
+      const int pieces = wave_total(units * ((s.steps + len - 1) / len));
+      if (pieces == tiles ||
+          plain_us(tiles, work, longest, p.slots, D) <= split_us(pieces, tiles, work, len, p.slots, D))
+        len = kPfWhole;
     }
     if (blockIdx.x == 0 && threadIdx.x == 0) *p.piece_len = len;
   }
-  s.n = (s.steps + len - 1) / len;
+  s.whole = len == kPfWhole;
+  s.n = s.whole ? 1 : (s.steps + len - 1) / len;
   const int mine = units * s.n;
   const int sum = wave_scan(mine);
   s.first = sum - mine;
@@ -272,10 +315,14 @@ __global__ __launch_bounds__(kPfThreads, 2) void paged_prefill_attn(PrefillParam
   // Balanced launch: XCD x takes the x-th eighth of the pieces.
   const int i = blockIdx.x;
   const int j = i / kPfXcds;
-  const int share = (j / p.share_tiles) * kPfXcds + i % kPfXcds;
-  const int u = share / p.spread;
-  const int jj = (j % p.share_tiles) * p.spread + share % p.spread;
-  if (!kSplit && (u >= p.units || jj >= p.tiles_per_unit)) return;
+  int u = 0, jj = 0;  // unit and place among its tiles; false where the grid has none
+  auto plain_item = [&]() {
+    const int share = (j / p.share_tiles) * kPfXcds + i % kPfXcds;
+    u = share / p.spread;
+    jj = (j % p.share_tiles) * p.spread + share % p.spread;
+    return u < p.units && jj < p.tiles_per_unit;
+  };
+  if (!kSplit && !plain_item()) return;
   // kPair: a workgroup takes row tiles n - 1 - jj and then jj (half of the workgroups
   // end at once) where the prompts are of about one length; in ragged batches the pairs
   // would be uneven.
@@ -290,23 +337,31 @@ __global__ __launch_bounds__(kPfThreads, 2) void paged_prefill_attn(PrefillParam
   int piece = 0, s0 = 0, s1 = 0;  // kSplit: the piece and its steps of the tile
   bool whole = true;
   if constexpr (kSplit) {
-    const SeqPieces seqs = seq_pieces<false>(p);
-    const int per_xcd = (seqs.total + kPfXcds - 1) / kPfXcds;
-    piece = (i % kPfXcds) * per_xcd + j;
-    if (j >= per_xcd || piece >= min(seqs.total, p.max_pieces)) return;
-    // The last sequence whose first piece is not past this one (sequences without
-    // queries share their successor's first, so it is the one that holds it).
-    b = 63 - __builtin_clzll(__ballot(static_cast<int>(threadIdx.x & 63) < p.batch && seqs.first <= piece));
-    const int in_seq = piece - __builtin_amdgcn_readlane(seqs.first, b);
-    const int tiles = __builtin_amdgcn_readlane(seqs.tiles, b);
-    const int steps = __builtin_amdgcn_readlane(seqs.steps, b);
-    const int n = __builtin_amdgcn_readlane(seqs.n, b);
-    kh = in_seq / (tiles * n);
-    const int x = in_seq / tiles % n;
-    tile = in_seq % tiles;
-    s0 = static_cast<int>(static_cast<int64_t>(steps) * x / n);
-    s1 = static_cast<int>(static_cast<int64_t>(steps) * (x + 1) / n);
-    whole = n == 1;
+    const SeqPieces seqs = seq_pieces<false, D>(p);
+    if (seqs.whole) {  // as the plain grid
+      if (!plain_item()) return;
+      tile = p.tiles_per_unit - 1 - jj;
+      b = u / p.num_kv_heads;
+      kh = u % p.num_kv_heads;
+      s1 = 1 << 24;
+    } else {
+      const int per_xcd = (seqs.total + kPfXcds - 1) / kPfXcds;
+      piece = (i % kPfXcds) * per_xcd + j;
+      if (j >= per_xcd || piece >= min(seqs.total, p.max_pieces)) return;
+      // The last sequence whose first piece is not past this one (sequences without
+      // queries share their successor's first, so it is the one that holds it).
+      b = 63 - __builtin_clzll(__ballot(static_cast<int>(threadIdx.x & 63) < p.batch && seqs.first <= piece));
+      const int in_seq = piece - __builtin_amdgcn_readlane(seqs.first, b);
+      const int tiles = __builtin_amdgcn_readlane(seqs.tiles, b);
+      const int steps = __builtin_amdgcn_readlane(seqs.steps, b);
+      const int n = __builtin_amdgcn_readlane(seqs.n, b);
+      kh = in_seq / (tiles * n);
+      const int x = in_seq / tiles % n;
+      tile = in_seq % tiles;
+      s0 = static_cast<int>(static_cast<int64_t>(steps) * x / n);
+      s1 = static_cast<int>(static_cast<int64_t>(steps) * (x + 1) / n);
+      whole = n == 1;
+    }
   } else {
     tile = pass == 0 ? p.tiles_per_unit - 1 - jj : jj;
     if (pass == 1) {
@@ -752,7 +807,8 @@ __global__ __launch_bounds__(256) void paged_prefill_merge(PrefillParams p) {
   constexpr int TPR = D / 4;             // threads per row
   constexpr int RPP = 256 / TPR;         // rows per pass
   constexpr int PARTS = kPfRows / kPfMergeRows;
-  const SeqPieces seqs = seq_pieces<true>(p);
+  const SeqPieces seqs = seq_pieces<true, D>(p);
+  if (seqs.whole) return;
   const int part = blockIdx.x % PARTS;
   const int x = blockIdx.x / PARTS;
   const int b = x / (p.num_kv_heads * p.tiles_per_unit);
@@ -814,34 +870,48 @@ __global__ __launch_bounds__(256) void paged_prefill_merge(PrefillParams p) {
 
 int64_t ceil_div64(int64_t a, int64_t b) { return (a + b - 1) / b; }
 
-// The most pieces of the balanced launch, 0 = the plain grid.
-// Long cached contexts only (causal rows of a whole prompt carry unequal keys).  A step
-// (128 rows x 64 keys, D = 128) takes about 1.03 us with one workgroup on a CU and 1.9
-// us with two; the pieces' fp32 rows and the merge add ~15 % and ~6 us.  Taken where
-// that beats the plain grid; a batch is expected to be ragged, so that it has ~15 %
-// less work than its longest sequence says.  Measured, plain -> balanced: two chunks of
-// 342-512 tokens behind 16k-24k keys 390 -> 310 us, 512 behind 8k 162 -> 87, 64 behind
-// 32k 586 -> 61, 16 x 16 behind 4k-8k 156 -> 92; left alone: 1024 behind 2k (64 vs 67
-// split), 2048 behind 8k (297 vs 316).
-int balanced_pieces(int64_t batch, int64_t num_heads, int64_t num_kv_heads, int64_t head_dim, int64_t max_seqlen_q,
+// The balanced launch's most pieces, 0 = the plain grid, and whether the kernel has to ask
+// the real lengths if cutting pays.
+// Long cached contexts only (causal rows of a whole prompt carry unequal keys).  Taken
+// where cutting pays with every sequence as long as the longest: two chunks of 342-512
+// tokens behind 16k-24k keys 390 -> 310 us, 512 behind 8k 147 -> 85, 64 behind 32k 513 ->
+// 62, 16 x 16 behind 4k-8k 149 -> 93, 4 x 256 behind 8k at D = 64 104 -> 91; left alone:
+// 1024 behind 2k (64 vs 67 split), 2048 behind 8k (297 vs 316).  Other batches may still
+// gain by being ragged, which only the kernel sees (15 of 20-118 behind 1k-8k 186 -> 150
+// us, 4 x 256 behind 1k-4k 71 -> 62); where it then cuts no tile, looking costs up to 4 us
+// (20 x 128 behind 6k-8k 335 -> 339, 7 x 256 behind 4k at D = 64 78.5 -> 82) with more
+// tiles than CUs and below 1 with fewer (4 x 256 behind 4k 80), so that it is done from
+// 200 and 60 us on.
+struct BalancedPlan {
+  int pieces = 0;
+  bool ask = false;
+};
+BalancedPlan balanced_plan(int64_t batch, int64_t num_heads, int64_t num_kv_heads, int64_t head_dim, int64_t max_seqlen_q,
                     int64_t max_seqlen_k, int64_t window_left) {
   if (batch <= 0 || batch > kPfSplitBatch || max_seqlen_q <= 0 || num_kv_heads <= 0 || num_heads < num_kv_heads ||
       num_heads / num_kv_heads > kPfRows || max_seqlen_k < 2 * max_seqlen_q || max_seqlen_k > INT32_MAX / 2)
-    return 0;
+    return {};
   const int64_t cus = oxide::device_cu_count();
   const int64_t slots = 2 * cus;
   const int64_t tpw = kPfRows / (num_heads / num_kv_heads);
   const int64_t tiles = batch * num_kv_heads * ceil_div64(max_seqlen_q, tpw);
-  if (tiles > 2 * slots) return 0;
+  if (tiles > 2 * slots) return {};
   const int64_t w = window_left < 0 || window_left >= max_seqlen_k ? -1 : window_left;
   const int64_t steps = steps_per_tile(static_cast<int>(max_seqlen_k), static_cast<int>(w), static_cast<int>(tpw));
   const int64_t pieces = std::min(2 * slots, tiles * ceil_div64(steps, kPfMinPiece));
-  if (pieces <= tiles || tiles * steps > INT32_MAX / 2) return 0;  // the kernel sums steps in 32 bits
-  const double unit = head_dim / 128.0;
-  const double plain = unit * ceil_div64(tiles, slots) * steps * (tiles > cus ? 1.9 : 1.03);
-  const double split =
-      std::max(unit * tiles * steps / slots * 1.9 * 1.15, unit * kPfMinPiece * 1.03) * (batch > 1 ? 0.85 : 1.0) + 6.0;
-  return split < plain ? static_cast<int>(pieces) : 0;
+  if (pieces <= tiles || tiles * steps > INT32_MAX / 2) return {};  // the kernel sums steps in 32 bits
+  // With equal lengths: the piece length the kernel would choose.
+  const int t = static_cast<int>(tiles), n = static_cast<int>(steps), d = static_cast<int>(head_dim);
+  auto equal = [&](int64_t most) {
+    return std::max<int64_t>(kPfMinPiece, ceil_div64(n, std::max<int64_t>(most / tiles, 1)));
+  };
+  int64_t len = equal(pieces);
+  if (pieces > slots && tiles <= slots && 8 * equal(slots) <= 18 * len) len = equal(slots);
+  const int cut = static_cast<int>(tiles * ceil_div64(n, len)), w0 = static_cast<int>(tiles * steps);
+  const float plain = plain_us(t, w0, n, static_cast<int>(slots), d);
+  const bool pays = cut > t && split_us(cut, t, w0, static_cast<int>(len), static_cast<int>(slots), d) < plain;
+  if (!pays && (batch == 1 || plain < (tiles <= cus ? 60.f : 200.f))) return {};
+  return {static_cast<int>(pieces), !pays};
 }
 size_t balanced_rows_bytes(int pieces, int64_t head_dim) {
   return static_cast<size_t>(pieces) * kPfRows * static_cast<size_t>(head_dim) * sizeof(float);
@@ -871,8 +941,9 @@ void launch_mode(const PrefillParams& p, dim3 grid, hipStream_t s) {
 }
 
 template <class Tag, int D>
-void launch_balanced(const PrefillParams& p, hipStream_t s) {
-  const dim3 grid(static_cast<unsigned>(ceil_div64(p.max_pieces, kPfXcds) * kPfXcds));
+void launch_balanced(const PrefillParams& p, unsigned plain, hipStream_t s) {
+  // Workgroups for the most pieces and, where no tile is cut, for the plain grid.
+  const dim3 grid(std::max(plain, static_cast<unsigned>(ceil_div64(p.max_pieces, kPfXcds) * kPfXcds)));
   if (p.block_table == nullptr)
     hipLaunchKernelGGL((paged_prefill_attn<Tag, D, kContiguous, false, false, true>), grid, dim3(kPfThreads), 0, s, p);
   else if (p.block_size % kPfKeys == 0)
@@ -894,11 +965,11 @@ void launch_prefix_mode(const PrefillParams& p, dim3 grid, hipStream_t s) {
 
 template <class Tag>
 bool launch_prefill(const PrefillParams& p, int head_dim, hipStream_t s) {
+  const dim3 grid(static_cast<unsigned>(ceil_div64(int64_t{p.units} * p.spread, kPfXcds) * kPfXcds * p.share_tiles));
   if (p.max_pieces > 0) {
-    head_dim == 128 ? launch_balanced<Tag, 128>(p, s) : launch_balanced<Tag, 64>(p, s);
+    head_dim == 128 ? launch_balanced<Tag, 128>(p, grid.x, s) : launch_balanced<Tag, 64>(p, grid.x, s);
     return true;
   }
-  const dim3 grid(static_cast<unsigned>(ceil_div64(int64_t{p.units} * p.spread, kPfXcds) * kPfXcds * p.share_tiles));
   if (head_dim == 128) {
     launch_mode<Tag, 128>(p, grid, s);
     return true;
@@ -1002,9 +1073,11 @@ void prefill_impl(void* out, const void* q, const void* k, const void* v, const 
   p.scale_log2 = softmax_scale * 1.4426950408889634f;
   p.batch = static_cast<int>(batch);
   if (workspace != nullptr && oxide::aligned16(workspace)) {
-    const int pieces = balanced_pieces(batch, num_heads, num_kv_heads, head_dim, max_seqlen_q, max_seqlen_k, window_left);
+    const auto [pieces, ask] =
+        balanced_plan(batch, num_heads, num_kv_heads, head_dim, max_seqlen_q, max_seqlen_k, window_left);
     if (pieces > 0 && workspace_bytes >= balanced_bytes(pieces, head_dim)) {
       p.max_pieces = pieces;
+      p.may_be_whole = ask;
       p.slots = 2 * oxide::device_cu_count();
       p.part_o = static_cast<float*>(workspace);
       p.part_lse = reinterpret_cast<float*>(static_cast<char*>(workspace) + balanced_rows_bytes(pieces, head_dim));
@@ -1044,7 +1117,8 @@ extern "C" size_t prefill_attention_workspace_size(int64_t batch, int64_t num_he
                                                          int64_t head_dim, int64_t max_seqlen_q, int64_t max_seqlen_k,
                                                          int32_t window_left) {
   if (head_dim != 64 && head_dim != 128) return 0;
-  const int pieces = balanced_pieces(batch, num_heads, num_kv_heads, head_dim, max_seqlen_q, max_seqlen_k, window_left);
+  const int pieces =
+      balanced_plan(batch, num_heads, num_kv_heads, head_dim, max_seqlen_q, max_seqlen_k, window_left).pieces;
   return pieces > 0 ? balanced_bytes(pieces, head_dim) : 0;
 }
 
