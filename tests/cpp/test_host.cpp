@@ -647,6 +647,91 @@ static void test_gpu_prefill_step() {
   for (void* ptr : {dk, dv, ds, dqkv, dq, dout, dcs}) (void)hipFree(ptr);
 }
 
+// One PrefillStep's layers on two streams, behind a context long enough to have its keys
+// split: the first stream's calls use the step's workspace, the other's must not (they
+// are the plain entry, bit for bit), whether one after the other or at the same time.
+static void test_gpu_prefill_step_streams() {
+  const std::size_t Hq = 8, H = 2, D = 64, BS = 64, P = 1500, T = 3, L = P + T, NB = (L + BS - 1) / BS;
+  PagedKVCache cache(2, NB, BS, H, D, OXIDE_DTYPE_BF16);
+  uint64_t s = 99;
+  auto rnd = [&s]() {
+    s = s * 6364136223846793005ULL + 1442695040888963407ULL;
+    return static_cast<float>(static_cast<int64_t>(s >> 11) % 2000 - 1000) / 500.f;
+  };
+  std::vector<uint16_t> kv(NB * BS * H * D), qkv(T * (Hq + 2 * H) * D);
+  for (auto& x : qkv) x = f2bf(rnd());
+  for (auto& x : kv) x = f2bf(rnd());
+  for (std::size_t layer = 0; layer < 2; ++layer) {
+    (void)hipMemcpy(cache.k_cache(layer), kv.data(), kv.size() * 2, hipMemcpyHostToDevice);
+    (void)hipMemcpy(cache.v_cache(layer), kv.data(), kv.size() * 2, hipMemcpyHostToDevice);
+  }
+  std::vector<int32_t> table;
+  for (std::size_t i = 0; i < NB; ++i) table.push_back(static_cast<int32_t>(i));
+  std::vector<int64_t> slots;
+  for (std::size_t t = 0; t < T; ++t) slots.push_back(static_cast<int64_t>(P + t));
+  const std::vector<float> cs = rope_cos_sin_cache(8, D, 1e6f);
+  const std::vector<uint32_t> cu = {0, T, 0, L};
+  void *dqkv, *dcs, *dcu, *dtab, *dq[2], *dout[2], *dplain;
+  (void)hipMalloc(&dqkv, qkv.size() * 2);
+  (void)hipMalloc(&dcs, cs.size() * 4);
+  (void)hipMalloc(&dcu, cu.size() * 4);
+  (void)hipMalloc(&dtab, table.size() * 4);
+  (void)hipMalloc(&dplain, T * Hq * D * 2);
+  for (int i = 0; i < 2; ++i) {
+    (void)hipMalloc(&dq[i], T * Hq * D * 2);
+    (void)hipMalloc(&dout[i], T * Hq * D * 2);
+  }
+  (void)hipMemcpy(dqkv, qkv.data(), qkv.size() * 2, hipMemcpyHostToDevice);
+  (void)hipMemcpy(dcs, cs.data(), cs.size() * 4, hipMemcpyHostToDevice);
+  (void)hipMemcpy(dcu, cu.data(), cu.size() * 4, hipMemcpyHostToDevice);
+  (void)hipMemcpy(dtab, table.data(), table.size() * 4, hipMemcpyHostToDevice);
+  const float scale = 0.125f;
+  CHECK(prefill_attention_workspace_size(1, Hq, H, D, T, L, -1) > 0);
+  hipStream_t st[2];
+  for (auto& x : st) CHECK(hipStreamCreate(&x) == hipSuccess);
+  PrefillStep step(cache, Hq);
+  step.upload(build_prefill_metadata({static_cast<uint32_t>(T)}, {static_cast<uint32_t>(L)}, slots), {table},
+              std::vector<int32_t>(T, 0), st[0]);
+  CHECK(hipStreamSynchronize(st[0]) == hipSuccess);
+  auto layer = [&](int i) {
+    step.run_layer(i, dqkv, nullptr, nullptr, 1e-6, static_cast<const float*>(dcs), 8, dq[i], dout[i], scale, -1,
+                   st[i]);
+  };
+  std::vector<uint16_t> out[2], plain(T * Hq * D);
+  auto fetch = [&](int i) {
+    out[i].assign(T * Hq * D, 0);
+    (void)hipMemcpy(out[i].data(), dout[i], out[i].size() * 2, hipMemcpyDeviceToHost);
+  };
+  for (int i = 0; i < 2; ++i) {
+    layer(i);
+    CHECK(hipDeviceSynchronize() == hipSuccess);
+    fetch(i);
+  }
+  ::paged_prefill_attention(dplain, dq[1], cache.k_cache(1), cache.v_cache(1), static_cast<const uint32_t*>(dcu),
+                            static_cast<const uint32_t*>(dcu) + 2, static_cast<const int32_t*>(dtab), NB, NB, 1, Hq, H,
+                            D, BS, T, L, -1, scale, OXIDE_DTYPE_BF16, nullptr);
+  CHECK(oxide_last_error() == OXIDE_OK);
+  (void)hipMemcpy(plain.data(), dplain, plain.size() * 2, hipMemcpyDeviceToHost);
+  CHECK(out[1] == plain);
+  CHECK(out[0] != plain);  // it was split
+  double max_err = 0;
+  for (std::size_t i = 0; i < plain.size(); ++i)
+    max_err = std::max(max_err, static_cast<double>(std::fabs(bf2f(out[0][i]) - bf2f(plain[i]))));
+  CHECK(max_err <= 2e-2);
+  const std::vector<uint16_t> split = out[0];
+  for (int n = 0; n < 20; ++n) {
+    layer(0);
+    layer(1);
+  }
+  CHECK(hipDeviceSynchronize() == hipSuccess);
+  fetch(0);
+  fetch(1);
+  CHECK(out[0] == split);
+  CHECK(out[1] == plain);
+  for (auto& x : st) (void)hipStreamDestroy(x);
+  for (void* p : {dqkv, dcs, dcu, dtab, dq[0], dq[1], dout[0], dout[1], dplain}) (void)hipFree(p);
+}
+
 // The fast divide of the attention prologue (exact_div.hpp) against the
 // correctly rounded x / b.  The quotient's significand depends only on the
 // significands of x and b while every step stays normal, so checking every
@@ -729,6 +814,7 @@ int main(int argc, char** argv) {
     test_gpu_append_known_answer();
     test_gpu_cow_all_layers();
     test_gpu_prefill_step();
+    test_gpu_prefill_step_streams();
     test_gpu_decode_step();
     test_gpu_decode_step_shared_prefix();
   } else {

@@ -246,7 +246,8 @@ void PrefillStep::upload(const AttnMetadata& meta, const std::vector<std::vector
     check(hipMalloc(&d_buf_, total), "hipMalloc(PrefillStep)");
     cap_ = total;
   }
-  // The unwindowed size covers every window.
+  ws_taken_ = false;
+  // The unwindowed size; a windowed call that wanted more would attend without it.
   const std::size_t ws = prefill_attention_workspace_size(
       static_cast<int64_t>(batch_), static_cast<int64_t>(num_heads_), static_cast<int64_t>(cache_.num_kv_heads()),
       static_cast<int64_t>(cache_.head_dim()), static_cast<int64_t>(max_seqlen_q_),
@@ -270,6 +271,19 @@ void PrefillStep::upload(const AttnMetadata& meta, const std::vector<std::vector
         "upload slot_mapping");
 }
 
+bool PrefillStep::owns_workspace(hipStream_t stream) {
+  // One handle, a stream per thread; a graph may be replayed beside the step's calls.
+  if (!d_ws_ || stream == hipStreamPerThread) return false;
+  hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(stream, &capture) != hipSuccess) (void)hipGetLastError();
+  if (capture != hipStreamCaptureStatusNone) return false;
+  if (!ws_taken_) {
+    ws_taken_ = true;
+    ws_stream_ = stream;
+  }
+  return ws_stream_ == stream;
+}
+
 void PrefillStep::run_layer(std::size_t layer, const void* qkv, const void* q_norm_weight,
                             const void* k_norm_weight, double eps, const float* cos_sin,
                             std::size_t max_position, void* q_scratch, void* out, float softmax_scale,
@@ -284,12 +298,16 @@ void PrefillStep::run_layer(std::size_t layer, const void* qkv, const void* q_no
                            cache_.v_cache(layer), reinterpret_cast<const int64_t*>(d + off_slots_),
                            static_cast<int64_t>(num_tokens_), Hq, Hkv, D, cache_.dtype(), stream);
   check_lib("qk_norm_rope_and_cache");
+  std::unique_lock<std::mutex> lock(ws_mutex_);
+  const bool split = owns_workspace(stream);
+  if (!split) lock.unlock();
   ::paged_prefill_attention_workspace(
       out, q_scratch, cache_.k_cache(layer), cache_.v_cache(layer), reinterpret_cast<const uint32_t*>(d),
       reinterpret_cast<const uint32_t*>(d + off_cuk_), reinterpret_cast<const int32_t*>(d + off_table_),
       static_cast<int64_t>(max_blocks_), static_cast<int64_t>(cache_.num_blocks()), static_cast<int64_t>(batch_), Hq,
       Hkv, D, static_cast<int64_t>(cache_.block_size()), static_cast<int64_t>(max_seqlen_q_),
-      static_cast<int64_t>(max_seqlen_k_), window_left, softmax_scale, d_ws_, cap_ws_, cache_.dtype(), stream);
+      static_cast<int64_t>(max_seqlen_k_), window_left, softmax_scale, split ? d_ws_ : nullptr, split ? cap_ws_ : 0,
+      cache_.dtype(), stream);
   check_lib("paged_prefill_attention_workspace");
 }
 

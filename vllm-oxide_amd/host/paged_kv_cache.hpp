@@ -11,6 +11,8 @@
 
 #include <hip/hip_runtime.h>
 
+#include <mutex>
+
 #include "oxide_host.hpp"
 #include "oxide_paged_kv.h"
 
@@ -128,6 +130,10 @@ class PrefillStep {
   // Layer `layer`: qkv [T, (Hq + 2 Hkv) D] -> q_scratch [T, Hq, D] (normed,
   // rotated), K/V appended at the slot mapping, out [T, Hq, D].  Norm weights
   // may be null (no q/k norm); cos_sin is the fp32 [max_position, D] table.
+  // Calls of one step may come from several streams and threads.  The workspace for keys
+  // split behind a long cached context goes with the stream of the first call after
+  // upload; calls on other streams, on hipStreamPerThread and under capture attend
+  // without it (paged_prefill_attention, the same result within rounding).
   void run_layer(std::size_t layer, const void* qkv, const void* q_norm_weight, const void* k_norm_weight,
                  double eps, const float* cos_sin, std::size_t max_position, void* q_scratch, void* out,
                  float softmax_scale, int32_t window_left, hipStream_t stream);
@@ -143,8 +149,13 @@ class PrefillStep {
   std::vector<int64_t> h_slots_;
   void* d_buf_ = nullptr;  // cu_q | cu_k | table | positions | slots, 256-byte aligned parts
   std::size_t cap_ = 0;
+  // Whether the workspace is this stream's (ws_mutex_ held).
+  bool owns_workspace(hipStream_t stream);
   void* d_ws_ = nullptr;  // partial rows of calls behind a long cached context
   std::size_t cap_ws_ = 0;
+  std::mutex ws_mutex_;  // held over a call that uses it: its two launches stay together
+  bool ws_taken_ = false;
+  hipStream_t ws_stream_ = nullptr;  // whose it is, once taken
   std::size_t off_cuk_ = 0, off_table_ = 0, off_pos_ = 0, off_slots_ = 0;
 };
 
