@@ -89,6 +89,38 @@ def test_library_errors_raise_through_the_native_calls(device):
             ox.prefill_attn(q, k, k, i32(0, 1), i32(0, 5), 1, 5, 0.1, i32(0)[None])
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("general", [False, True], ids=["native", "general"])
+def test_prefill_without_room_for_a_workspace(device, general, monkeypatch):
+    """A prefill call whose workspace does not fit into the memory left attends without one."""
+    if general:
+        _general(monkeypatch)
+    g = torch.Generator(device=device).manual_seed(5)
+    rnd = lambda *s: torch.randn(s, generator=g, device=device, dtype=torch.bfloat16)  # noqa: E731
+    i32 = lambda *v: torch.tensor(v, dtype=torch.int32, device=device)  # noqa: E731
+    q, k, v = rnd(512, 32, 128), rnd(8192, 8, 128), rnd(8192, 8, 128)
+    out = torch.empty_like(q)
+    cq, ck = i32(0, 512), i32(0, 8192)
+    L = ox.load()
+    need = L.prefill_attention_workspace_size(1, 32, 8, 128, 512, 8192, -1)
+    assert need > 30 << 20
+    call = lambda o: ox.prefill_attn(q, k, v, cq, ck, 512, 8192, 0.09, out=o)  # noqa: E731
+    want = torch.empty_like(out)
+    L.varlen_prefill_attention(want.data_ptr(), q.data_ptr(), k.data_ptr(), v.data_ptr(), cq.data_ptr(), ck.data_ptr(),
+                               8192, 1, 32, 8, 128, 512, 8192, -1, 0.09, 1, torch.cuda.current_stream().cuda_stream)
+    torch.cuda.synchronize()
+    torch.cuda.empty_cache()
+    total = torch.cuda.get_device_properties(device).total_memory
+    try:
+        torch.cuda.set_per_process_memory_fraction((torch.cuda.memory_reserved(device) + (1 << 20)) / total, device)
+        assert call(out) is out
+    finally:
+        torch.cuda.set_per_process_memory_fraction(1.0, device)
+    torch.cuda.synchronize()
+    assert torch.equal(out, want)
+    assert not torch.equal(call(torch.empty_like(out)), want)  # with a workspace its keys are split
+
+
 def test_host_tensors_are_refused_alike(monkeypatch):
     s = _inputs("cpu")
     calls = [lambda: ox.decode_attn(s["q"], s["k"], s["v"], s["cu"], s["table"], 130, 0.1, page_block_size=64),

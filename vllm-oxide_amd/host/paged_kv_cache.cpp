@@ -256,8 +256,12 @@ void PrefillStep::upload(const AttnMetadata& meta, const std::vector<std::vector
     if (d_ws_) check(hipFree(d_ws_), "hipFree");
     d_ws_ = nullptr;
     cap_ws_ = 0;
-    check(hipMalloc(&d_ws_, ws), "hipMalloc(PrefillStep)");
-    cap_ws_ = ws;
+    if (hipMalloc(&d_ws_, ws) == hipSuccess) {
+      cap_ws_ = ws;
+    } else {  // no room: the calls attend without it
+      (void)hipGetLastError();
+      d_ws_ = nullptr;
+    }
   }
   char* d = static_cast<char*>(d_buf_);
   check(hipMemcpyAsync(d, h_cuq_.data(), h_cuq_.size() * 4, hipMemcpyHostToDevice, stream), "upload cu_seqlens_q");

@@ -259,7 +259,10 @@ def prefill_attn(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, cu_seqlens_q
     w = -1 if window_left is None else int(window_left)
     Hkv = k.shape[-2]
     need = int(L.prefill_attention_workspace_size(B, Hq, Hkv, D, max_seqlen_q, max_seqlen_k, w))
-    workspace = torch.empty(need, dtype=torch.uint8, device=q.device) if need else None
+    try:
+        workspace = torch.empty(need, dtype=torch.uint8, device=q.device) if need else None
+    except torch.cuda.OutOfMemoryError:  # it attends without one
+        workspace, need = None, 0
     if block_table is not None:
         NB, BS, Hkv, D2 = k.shape
         if D2 != D or block_table.dtype != torch.int32:

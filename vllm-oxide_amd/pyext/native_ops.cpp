@@ -153,9 +153,13 @@ PyObject* prefill(PyObject*, PyObject* const* a, Py_ssize_t n) {
     Py_RETURN_NONE;
   const int64_t B = cq->size(0) - 1, Hq = q->size(1), D = q->size(2), Hkv = k->size(kd - 2);
   at::Tensor o = out ? *out : at::empty_like(*q);
-  const size_t need = g_prefill_ws(B, Hq, Hkv, D, max_q, max_k, window);
+  size_t need = g_prefill_ws(B, Hq, Hkv, D, max_q, max_k, window);
   at::Tensor w;
-  if (need > 0) w = bytes_like(*q, static_cast<int64_t>(need));
+  try {
+    if (need > 0) w = bytes_like(*q, static_cast<int64_t>(need));
+  } catch (const c10::OutOfMemoryError&) {  // it attends without one
+    need = 0;
+  }
   void* s = stream_of(*q);
   void *po = o.data_ptr(), *pq = q->data_ptr(), *pk = k->data_ptr(), *pv = v->data_ptr();
   void* pw = need > 0 ? w.data_ptr() : nullptr;
