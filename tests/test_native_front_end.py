@@ -1,7 +1,11 @@
-"""The ops' native front end (_native.so) against the general Python code it stands in for:
+"""The ops' native front end (_native) against the general Python code it stands in for:
 the same outputs bit for bit over the argument forms it takes and those it leaves, and the
 same errors."""
+import importlib.util
 import math
+import subprocess
+import sys
+from pathlib import Path
 
 import numpy as np
 import pytest
@@ -10,6 +14,7 @@ import torch
 import oxide_paged_kv as ox
 from oxide_paged_kv import ops
 
+REPO = Path(__file__).resolve().parent.parent
 
 def _general(monkeypatch):
     """ops with the native front end declining every call."""
@@ -138,3 +143,73 @@ def test_host_tensors_are_refused_alike(monkeypatch):
                 call()
             messages.append(str(e.value))
     assert messages[:len(calls)] == messages[len(calls):]
+
+
+_STEP = """
+import sys
+sys.path[:0] = [{root!r}, {pkg!r}]
+{before}
+import torch
+import oxide_paged_kv as ox
+from oxide_paged_kv import _lib, ops
+ox.load()
+assert _lib._native is None
+q = torch.zeros(1, 4, 128, dtype=torch.bfloat16)
+k = torch.zeros(2, 64, 2, 128, dtype=torch.bfloat16)
+i = torch.tensor([0, 5], dtype=torch.int32)
+try:
+    ox.decode_attn(q, k, k, i, i[None], 5, 0.1, page_block_size=64)
+except ox.OxideError as e:
+    print("general:", e)
+"""
+
+
+@pytest.mark.parametrize("before", ["sys.modules['oxide_paged_kv._native'] = None",
+                                    "import torch; torch.__version__ += '.other'"], ids=["absent", "other-torch"])
+def test_package_works_without_the_native_module(before):
+    """No module (as after make), or one built against another torch: the general code runs."""
+    code = _STEP.format(root=str(REPO), pkg=str(REPO / "vllm-oxide_amd"), before=before)
+    r = subprocess.run([sys.executable, "-c", code], capture_output=True, text=True, timeout=120)
+    assert r.returncode == 0, r.stderr
+    assert r.stdout == "general: expected a device tensor\n"
+
+
+def _build_module():
+    spec = importlib.util.spec_from_file_location("oxide_build", REPO / "vllm-oxide_amd" / "build.py")
+    mod = importlib.util.module_from_spec(spec)
+    spec.loader.exec_module(mod)
+    return mod
+
+
+def test_c_libraries_are_linked_whatever_the_native_module_does(monkeypatch, tmp_path):
+    b = _build_module()
+    done = []
+
+    def run(cmd, **kw):
+        done.append("archive" if cmd[0] == "ar" else "link" if "-shared" in cmd else "compile")
+        return subprocess.CompletedProcess(cmd, 0, "", "")
+
+    def fails():
+        raise RuntimeError("no native module")
+
+    monkeypatch.setattr(b, "BUILD", tmp_path)
+    monkeypatch.setattr(b, "RESOURCES", tmp_path / "r.json")
+    monkeypatch.setattr(b, "LIB", tmp_path / "l.so")
+    monkeypatch.setattr(b, "STATIC_LIB", tmp_path / "l.a")
+    monkeypatch.setattr(b, "build_native", fails)
+    monkeypatch.setattr(b, "build_host_test", lambda: done.append("host test"))
+    monkeypatch.setattr(b.subprocess, "run", run)
+    with pytest.raises(RuntimeError, match="no native module"):
+        b.build()
+    assert done[-3:] == ["link", "archive", "host test"]
+
+
+def test_native_module_is_left_out_without_torch_or_compiler(monkeypatch, tmp_path, capsys):
+    b = _build_module()
+    monkeypatch.setattr(b, "NATIVE_LIB", tmp_path / b.NATIVE_LIB.name)
+    (tmp_path / "_native.so").write_bytes(b"stale")
+    monkeypatch.setattr(b.shutil, "which", lambda name: None)
+    assert b.build_native() is None and not list(tmp_path.iterdir())
+    monkeypatch.setitem(sys.modules, "torch", None)
+    assert b.build_native() is None
+    assert capsys.readouterr().err.count("native front end not built") == 2

@@ -5,14 +5,17 @@ cmake, no JIT cache), so the .so travels with the source tree.  Every call
 recompiles.  Counterpart of the reference's crates/vllm-oxide/build.rs:1-30
 (nvcc via cudaforge -> static lib); here hipcc --offload-arch=gfx950 -> the
 shared library Python loads with ctypes, plus the same objects archived as
-liboxide_paged_kv.a, and the Python ops' native module against torch's headers.  rust/oxide-paged-kv-sys/build.rs and
-vllm-oxide_amd/Makefile compile the same sources with the same flags.
+liboxide_paged_kv.a, and the Python ops' native module against torch's headers (where
+torch and g++ are there).  rust/oxide-paged-kv-sys/build.rs and vllm-oxide_amd/Makefile
+compile the same library sources with the same flags.
 """
 from __future__ import annotations
 
 import os
+import shutil
 import subprocess
 import sys
+import sysconfig
 from concurrent.futures import ThreadPoolExecutor
 from pathlib import Path
 
@@ -24,9 +27,10 @@ INCLUDE = REPO / "include"
 BUILD = PKG / "_build"
 LIB = PKG / "liboxide_paged_kv.so"
 STATIC_LIB = PKG / "liboxide_paged_kv.a"
-# The Python ops' native front end: a CPython module against torch's C++ headers.
+# The Python ops' native front end: a CPython module against torch's C++ headers, named
+# for the interpreter it is built for.
 NATIVE_SRC = PKG / "pyext" / "native_ops.cpp"
-NATIVE_LIB = PKG / "oxide_paged_kv" / "_native.so"
+NATIVE_LIB = PKG / "oxide_paged_kv" / f"_native{sysconfig.get_config_var('EXT_SUFFIX') or '.so'}"
 HOST_TEST_SRC = REPO / "tests" / "cpp" / "test_host.cpp"
 HOST_TEST_BIN = REPO / "tests" / "cpp" / "build" / "test_host"
 HOST_TEST_STAMP = HOST_TEST_BIN.with_suffix(".sources.sha256")
@@ -79,16 +83,24 @@ def _compile(src: Path):
     return obj, _parse_resources(r.stderr)
 
 
-def build_native() -> Path:
-    """oxide_paged_kv/_native.so with the host compiler; it links torch's libraries, which
-    `import torch` has loaded by then."""
-    import sysconfig
-
-    import torch
-
+def build_native() -> Path | None:
+    """The ops' native module with the host compiler; it links torch's libraries, which
+    `import torch` has loaded by then.  None without torch or g++: the ops then call the
+    library through ctypes only."""
+    for old in NATIVE_LIB.parent.glob("_native*.so"):  # never a module of earlier sources
+        old.unlink()
+    try:
+        import torch
+    except ImportError as e:
+        print(f"native front end not built: {e}", file=sys.stderr)
+        return None
+    if shutil.which("g++") is None:
+        print("native front end not built: no g++", file=sys.stderr)
+        return None
     t = Path(torch.__file__).resolve().parent
     cmd = ["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
-           f"-D_GLIBCXX_USE_CXX11_ABI={int(torch.compiled_with_cxx11_abi())}", "-I", str(INCLUDE),
+           f"-D_GLIBCXX_USE_CXX11_ABI={int(torch.compiled_with_cxx11_abi())}",
+           f'-DOXIDE_TORCH_VERSION="{torch.__version__}"', "-I", str(INCLUDE),
            "-isystem", str(t / "include"), "-isystem", str(t / "include" / "torch" / "csrc" / "api" / "include"),
            "-isystem", "/opt/rocm/include", "-isystem", sysconfig.get_paths()["include"], str(NATIVE_SRC),
            "-o", str(NATIVE_LIB), "-L", str(t / "lib"), "-ltorch_python", "-ltorch_cpu", "-lc10", "-lc10_hip"]
@@ -104,7 +116,6 @@ def build(verbose: bool = False) -> Path:
     with ThreadPoolExecutor(max_workers=min(9, len(srcs) + 1)) as ex:
         native = ex.submit(build_native)
         results = list(ex.map(_compile, srcs))
-        native.result()
     objs = [o for o, _ in results]
     import json
 
@@ -123,6 +134,7 @@ def build(verbose: bool = False) -> Path:
     if r.returncode != 0:
         raise RuntimeError(f"ar failed:\n{r.stdout}\n{r.stderr}")
     build_host_test()
+    native.result()  # last: the C libraries do not need it
     if verbose:
         print(f"built {LIB}")
     return LIB
@@ -162,5 +174,7 @@ def build_host_test() -> Path:
 
 
 if __name__ == "__main__":
+    if sys.argv[1:] == ["native"]:
+        sys.exit(0 if build_native() else 1)
     build(verbose=True)
     sys.exit(0)

@@ -1,7 +1,7 @@
 """MI355X (gfx950) paged-KV hot path of vllm-oxide: Python front end.
 
 The kernels live in liboxide_paged_kv.so (HIP, built in-tree by
-vllm-oxide_amd/build.py); this package binds them (ctypes, and _native.so for the
+vllm-oxide_amd/build.py); this package binds them (ctypes, and the native module _native for the
 calls of a serving step) and generates the synthetic workloads of the benchmark configurations.
 """
 from ._lib import LIB_PATH, OxideError, load  # noqa: F401

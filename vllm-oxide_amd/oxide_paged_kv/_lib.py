@@ -1,6 +1,8 @@
 """ctypes binding of include/oxide_paged_kv.h (liboxide_paged_kv.so).
 
-There is no fallback: if the HIP library is not built, importing the ops raises.
+There is no fallback for the HIP library: if it is not built, the first call raises.
+The native front end (_native, pyext/native_ops.cpp) is optional: without it the ops call
+the library through ctypes only.
 """
 from __future__ import annotations
 
@@ -8,7 +10,14 @@ import ctypes
 import os
 from pathlib import Path
 
-import torch  # noqa: F401  (its libraries first: _native links to them)
+import torch  # its libraries first: _native links to them
+
+try:
+    from . import _native
+except ImportError:  # not built (make builds the C libraries only), or for another interpreter
+    _native = None
+if _native is not None and _native.torch_version != torch.__version__:
+    _native = None  # built against another torch's headers
 
 PKG_DIR = Path(__file__).resolve().parent.parent
 # OXIDE_PAGED_KV_LIB points at another build of the same library (e.g. a tuning variant).
@@ -93,10 +102,7 @@ def load() -> ctypes.CDLL:
             fn = getattr(L, name)
             fn.restype = res
             fn.argtypes = args
-        # The native front end (_native.so, built beside the library) calls this library.
-        from . import _native
-
-        for name in SIGNATURES:
+        for name in SIGNATURES if _native is not None else ():  # the native front end calls this library
             _native.bind(name, ctypes.cast(getattr(L, name), ctypes.c_void_p).value)
         _lib = L
     return _lib

@@ -12,14 +12,27 @@
 Tensors must be contiguous CUDA (HIP) tensors; every call goes to the HIP library
 on torch's current stream and raises OxideError if the library reports an error.
 The calls of a serving step (decode, prefill, prologue, metadata) go through the native
-front end (_native.so, pyext/native_ops.cpp) when their arguments are of the plain form;
-the code here handles the other forms and raises the argument errors.
+front end (_native, pyext/native_ops.cpp) when it is built and their arguments are of the
+plain form; the code here handles the other forms and raises the argument errors.
 """
 from __future__ import annotations
 
 import torch
 
-from . import _lib, _native
+from . import _lib
+
+
+class _General:
+    """In the native front end's place where it is not built: declines every call."""
+
+    @staticmethod
+    def decode(*args):
+        return None
+
+    prefill = prologue = metadata = decode
+
+
+_native = _lib._native or _General
 
 _DTYPE_CODE = {torch.float16: _lib.DTYPE_F16, torch.bfloat16: _lib.DTYPE_BF16,
                torch.float32: _lib.DTYPE_F32}

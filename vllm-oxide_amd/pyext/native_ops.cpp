@@ -1,4 +1,4 @@
-// Native front end of the Python ops (oxide_paged_kv/_native.so): checks the tensors,
+// Native front end of the Python ops (oxide_paged_kv/_native, a CPython module): checks the tensors,
 // allocates outputs and workspaces through torch's allocator and calls the C ABI, for
 // the calls of a serving step.  ops.py calls these first; each returns
 //   * the op's result,
@@ -277,4 +277,9 @@ PyModuleDef kModule = {PyModuleDef_HEAD_INIT, "_native", nullptr, -1, kMethods, 
 
 }  // namespace
 
-PyMODINIT_FUNC PyInit__native() { return PyModule_Create(&kModule); }
+PyMODINIT_FUNC PyInit__native() {
+  PyObject* m = PyModule_Create(&kModule);
+  // The torch whose headers it was built against; _lib.py uses it with no other.
+  if (m && PyModule_AddStringConstant(m, "torch_version", OXIDE_TORCH_VERSION) < 0) Py_CLEAR(m);
+  return m;
+}
