@@ -120,6 +120,19 @@ def test_decode_many_splits_vs_oracle(device, case):
     assert_attn_close(got, oracle.paged_decode_attention(q, kc, vc, cu, table, 1.0 / math.sqrt(D), window, dtype))
 
 
+def test_decode_merge_of_more_than_64_splits_per_wave(device):
+    """1094 splits of one sequence: 69 for each of the merge's 16 waves, so that a wave's
+    log-sum-exps take a second round.  Scaled bar: a lost split would pass the absolute one."""
+    import oxide_paged_kv as ox
+
+    L = 140000
+    q, kc, vc, cu, table, mx = _case(17, 1, 2, 1, 64, 256, 550, [L], "bf16")
+    assert ox.split_tokens(1, 1, L) == 128 and -(-L // 128) > 16 * 64
+    print(f"decode merge of many splits L={L}", flush=True)
+    got = to_f32(_run(device, q, kc, vc, cu, table, mx, 0.125, -1, "bf16"))
+    assert_attn_scaled(got, oracle.paged_decode_attention(q, kc, vc, cu, table, 0.125, -1, "bf16"), label="many splits")
+
+
 def _random_shapes(seed, n):
     """Seeded random shapes over what the fixed cases combine separately: kv heads
     1/2/3/4/8, groups 1-8 and 16, D 64/128, page sizes 16/32/256, bf16/f16, ragged

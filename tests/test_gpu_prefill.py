@@ -400,3 +400,42 @@ def test_prefill_cuts_tiles_where_the_lengths_call_for_it(device, case):
     assert torch.equal(got, again)
     assert torch.equal(got, want) != cut
     assert_attn_close(to_f32(got), to_f32(want))
+
+
+@pytest.mark.parametrize("case", [BALANCED[2], BALANCED[4]], ids=["b2", "b4"])
+def test_prefill_workspace_forms(device, case):
+    """No workspace, a misaligned one and one a byte short are the plain call; the full one
+    is not written past its end.  The plain entries against the oracle too."""
+    import torch
+    from oxide_paged_kv import _lib
+
+    lq, lk, Hq, Hkv, D, BS, window, dtype = case
+    q, kc, vc, cuq, cuk, table = _case(87, lq, lk, Hq, Hkv, D, BS, dtype)
+    scale = 1.0 / math.sqrt(D)
+    need = _workspace_size(q, kc, cuq, cuk, window)
+    assert need > 0
+    print(f"prefill workspace forms lq={lq} lk={lk} window={window} {dtype}", flush=True)
+    args = (device, q, kc, vc, cuq, cuk, table, scale, window, dtype)
+    plain, _ = _entry(*args)
+    want = oracle.prefill_attention(q, kc, vc, cuq, cuk, scale, table, window, dtype)
+    assert_attn_close(to_f32(plain), want)
+    for size, offset in ((0, 0), (need, 4), (need - 1, 0)):
+        got, kept = _entry(*args, size, offset)
+        assert torch.equal(got, plain) and kept
+    got, kept = _entry(*args, need, 256)
+    assert kept and not torch.equal(got, plain)  # keys were split
+    assert_attn_close(to_f32(got), want)
+
+    # Contiguous K/V: the plain entry, and the workspace entry without one.
+    L = _lib.load()
+    t = lambda a: to_torch(a, dtype, device)  # noqa: E731
+    i32 = lambda a: torch.from_numpy(a.view(np.int32)).to(device)  # noqa: E731
+    qd, kd, vd, cq, ck = t(q), t(_contiguous(kc, cuk, table)), t(_contiguous(vc, cuk, table)), i32(cuq), i32(cuk)
+    code, stream = _lib.DTYPE_BF16 if dtype == "bf16" else _lib.DTYPE_F16, torch.cuda.current_stream().cuda_stream
+    for name, ws in (("varlen_prefill_attention", ()), ("varlen_prefill_attention_workspace", (None, 0))):
+        out = torch.zeros_like(qd)
+        getattr(L, name)(out.data_ptr(), qd.data_ptr(), kd.data_ptr(), vd.data_ptr(), cq.data_ptr(), ck.data_ptr(),
+                         kd.shape[0], len(lq), Hq, Hkv, D, max(lq), max(lk), window, scale, *ws, code, stream)
+        _lib.check()
+        torch.cuda.synchronize()
+        assert torch.equal(out, plain)

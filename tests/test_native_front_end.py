@@ -68,11 +68,30 @@ def _calls(s):
     return out + list(ox.build_decode_metadata(s["lens"], s["table"], BS))
 
 
+class _Counts:
+    """The native front end, noting which calls it took (True) and which it declined."""
+
+    def __init__(self, native):
+        self.native, self.taken = native, []
+
+    def __getattr__(self, name):
+        def call(*args):
+            r = getattr(self.native, name)(*args)
+            self.taken.append((name, r is not None))
+            return r
+        return call
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "f16"])
 def test_native_calls_equal_general_calls(device, dtype, monkeypatch):
     print(f"native front end {dtype}", flush=True)
+    counts = _Counts(ops._native)
+    monkeypatch.setattr(ops, "_native", counts)
     got = _calls(_inputs(device, dtype))
+    # Declined: the decode call with an append list and a numpy scale; return_k is not asked.
+    assert counts.taken == [("decode", True)] * 3 + [("decode", False), ("decode", True)] + \
+        [("prefill", True)] * 4 + [("prologue", True)] * 2 + [("metadata", True)]
     _general(monkeypatch)
     want = _calls(_inputs(device, dtype))
     torch.cuda.synchronize()
@@ -82,8 +101,10 @@ def test_native_calls_equal_general_calls(device, dtype, monkeypatch):
 
 
 @pytest.mark.gpu
-def test_library_errors_raise_through_the_native_calls(device):
+def test_library_errors_raise_through_the_native_calls(device, monkeypatch):
     """Errors the library records (a workspace-free shape check here: head size 96)."""
+    counts = _Counts(ops._native)
+    monkeypatch.setattr(ops, "_native", counts)
     q = torch.zeros(1, 4, 96, dtype=torch.bfloat16, device=device)
     k = torch.zeros(2, 64, 2, 96, dtype=torch.bfloat16, device=device)
     i32 = lambda *v: torch.tensor(v, dtype=torch.int32, device=device)  # noqa: E731
@@ -92,6 +113,7 @@ def test_library_errors_raise_through_the_native_calls(device):
             ox.decode_attn(q, k, k, i32(0, 5), i32(0)[None], 5, 0.1, page_block_size=64)
         with pytest.raises(ox.OxideError):
             ox.prefill_attn(q, k, k, i32(0, 1), i32(0, 5), 1, 5, 0.1, i32(0)[None])
+    assert counts.taken == [("decode", True), ("prefill", True)] * 2
 
 
 @pytest.mark.gpu
@@ -118,8 +140,13 @@ def test_prefill_without_room_for_a_workspace(device, general, monkeypatch):
     total = torch.cuda.get_device_properties(device).total_memory
     try:
         torch.cuda.set_per_process_memory_fraction((torch.cuda.memory_reserved(device) + (1 << 20)) / total, device)
+        held = []  # what the allocator still has of that size (after other tests)
+        with pytest.raises(torch.cuda.OutOfMemoryError):
+            while True:
+                held.append(torch.empty(need, dtype=torch.uint8, device=device))
         assert call(out) is out
     finally:
+        held = None
         torch.cuda.set_per_process_memory_fraction(1.0, device)
     torch.cuda.synchronize()
     assert torch.equal(out, want)
