@@ -38,10 +38,10 @@
 // on one XCD (workgroup i runs on XCD i % 8), so its K/V is fetched from HBM
 // once into that XCD's L2 and re-read from there; within a unit the tiles
 // with the most keys (last tokens) start first.  Where such units would load the XCDs
-// unevenly, each one's tiles alternate over 2, 4 or 8 of them (spread).  In large batches of short prompts of
-// about one length (kPair) a workgroup takes two row tiles of its unit, n - 1 - i and
-// then i; behind long cached contexts (kSplit) a row tile's keys are cut into pieces where
-that pays.
+// unevenly, each one's tiles alternate over 2, 4 or 8 of them (spread).  In large
+// batches of short prompts of about one length (kPair) a workgroup takes two row tiles
+// of its unit, n - 1 - i and then i; behind long cached contexts (kSplit) a row tile's
+// keys are cut into pieces where that pays.
 #include <math.h>
 
 #include <algorithm>
