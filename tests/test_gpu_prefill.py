@@ -377,7 +377,7 @@ REAL_LENGTHS = [
     ([256] * 8, [1024 + 438 * i for i in range(8)], True),        # 256 ragged ones
     ([128] * 40, [500] * 39 + [12000], True),                     # 640, one sequence far longer
     ([1024], [8704], True),                                       # pieces in one round
-    ([704, 1024], [4096, 6144], True),                            # and in two
+    ([704, 1024], [12288, 18432], True),                          # and in two (a third of it: as long whole)
 ]
 
 

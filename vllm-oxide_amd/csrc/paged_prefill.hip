@@ -174,13 +174,14 @@ __host__ __device__ __forceinline__ float plain_us(int tiles, int work, int long
   const float once = alone * longest + (both - alone) * (static_cast<float>(work) / tiles);
   return tiles > slots ? fmaxf(once, 1.25f * both * work / slots) : once;
 }
-// Each piece writes and the merge reads fp32 rows; the merge is a launch, and a piece
-// starts up as a tile does.
+// Each piece writes and the merge reads fp32 rows; the merge is a launch, and pieces in
+// two rounds start up twice (28 x 64 behind 1k-4k 112 us whole, 123 cut; 14 x 128 99 and
+// 110; 15 of 20-118 behind 0.5k-4k 103 and 88).
 __host__ __device__ __forceinline__ float split_us(int pieces, int tiles, int work, int len, int slots, int d) {
   const float alone = d == 128 ? 1.06f : 0.75f, both = d == 128 ? 1.9f : 1.1f;
   const float steps = 2 * pieces <= slots ? alone * len
                       : pieces <= slots   ? both * len
-                                          : both * (tiles > slots ? 1.6f : 1.15f) * work / slots;
+                                          : both * (tiles > slots ? 1.6f : 1.15f) * work / slots + 18.f;
   return steps + 1e-4f * d * pieces + 7.f;
 }
 constexpr int kPfWhole = INT32_MAX;  // the piece length stored where no tile is cut
@@ -190,7 +191,7 @@ constexpr int kPfWhole = INT32_MAX;  // the piece length stored where no tile is
 __device__ __forceinline__ int shortest_piece(int units, int steps, int slots, int tiles, int work) {
   // units * steps / len <= pieces <= units * (steps / len + 1) bound the bisection.
   int lo = max(kPfMinPiece, (work + slots - 1) / slots);
-  int hi = slots > tiles ? max(lo, (work + slots - tiles - 1) / (slots - tiles)) : INT32_MAX / 2;
+  int hi = max(lo, slots > tiles ? (work + slots - tiles - 1) / (slots - tiles) : wave_max(units > 0 ? steps : 0));
   while (lo < hi) {
     const int mid = (lo + hi) / 2;
     if (wave_total(units * ((steps + mid - 1) / mid)) <= slots)
@@ -433,11 +434,10 @@ __global__ __launch_bounds__(kPfThreads, 2) void paged_prefill_attn(PrefillParam
   }
   // The wave's own tiles [it0, it1): those in which some row of it sees a key (none
   // without rows).  The others it only loads for the rest.
-  const int wr0 = wave * 32;
-  const int wt_first = t0 + wr0 / G;
+  const int wt_first = __builtin_amdgcn_readlane(tq, 0);  // lanes 0 and 31 hold its first and last row
   int it0 = ntiles, it1 = ntiles;
-  if (wr0 < rows_used && wt_first < t1) {
-    const int wt_last = min(t1 - 1, t0 + min(wr0 + 31, rows_used - 1) / G);
+  if (wave * 32 < rows_used && wt_first < t1) {
+    const int wt_last = min(t1 - 1, __builtin_amdgcn_readlane(tq, 31));
     const int wave_hi = kPrefix ? khi : min(Lk - 1, wt_last + off);
     const int wave_lo = !kPrefix && W >= 0 ? wt_first + off - W : 0;
     it1 = wave_hi >= kt0 ? min(ntiles, (wave_hi - kt0) / kPfKeys + 1) : 0;
@@ -880,10 +880,10 @@ int64_t ceil_div64(int64_t a, int64_t b) { return (a + b - 1) / b; }
 // 62, 16 x 16 behind 4k-8k 149 -> 93, 4 x 256 behind 8k at D = 64 104 -> 91; left alone:
 // 1024 behind 2k (64 vs 67 split), 2048 behind 8k (297 vs 316).  Other batches may still
 // gain by being ragged, which only the kernel sees (15 of 20-118 behind 1k-8k 186 -> 150
-// us, 4 x 256 behind 1k-4k 71 -> 62); where it then cuts no tile, looking costs up to 4 us
-// (20 x 128 behind 6k-8k 335 -> 339, 7 x 256 behind 4k at D = 64 78.5 -> 82) with more
-// tiles than CUs and below 1 with fewer (4 x 256 behind 4k 80), so that it is done from
-// 200 and 60 us on.
+// us, 4 x 256 behind 1k-4k 71 -> 62, 7 of 30-252 behind 1k-8k at D = 64 148 -> 83); where
+// it then cuts no tile, looking costs up to 5 us (20 x 128 behind 6k-8k 330 -> 336, 14 x 128
+// behind 4k 120 -> 125, 4 x 256 behind 4k 74 -> 78.5), so that it is done from 200 us on
+// with more tiles than slots, 100 with more than CUs and 60 with fewer.
 struct BalancedPlan {
   int pieces = 0;
   bool ask = false;
@@ -912,7 +912,11 @@ BalancedPlan balanced_plan(int64_t batch, int64_t num_heads, int64_t num_kv_head
   const int cut = static_cast<int>(tiles * ceil_div64(n, len)), w0 = static_cast<int>(tiles * steps);
   const float plain = plain_us(t, w0, n, static_cast<int>(slots), d);
   const bool pays = cut > t && split_us(cut, t, w0, static_cast<int>(len), static_cast<int>(slots), d) < plain;
-  if (!pays && (batch == 1 || plain < (tiles <= cus ? 60.f : 200.f))) return {};
+  // Ragged: a sixth less work than equal lengths have.
+  const bool may = batch > 1 && plain >= (tiles <= cus ? 60.f : tiles <= slots ? 100.f : 200.f) &&
+                   (tiles > slots || 1.9 * 1.15 * 0.85 * tiles * steps / slots + 768.0 / d <
+                                         steps * (tiles > cus ? 1.9 : 1.03));
+  if (!pays && !may) return {};
   return {static_cast<int>(pieces), !pays};
 }
 size_t balanced_rows_bytes(int pieces, int64_t head_dim) {
