@@ -881,7 +881,7 @@ int64_t ceil_div64(int64_t a, int64_t b) { return (a + b - 1) / b; }
 // 1024 behind 2k (64 vs 67 split), 2048 behind 8k (297 vs 316).  Other batches may still
 // gain by being ragged, which only the kernel sees (15 of 20-118 behind 1k-8k 186 -> 150
 // us, 4 x 256 behind 1k-4k 71 -> 62, 7 of 30-252 behind 1k-8k at D = 64 148 -> 83); where
-// it then cuts no tile, looking costs up to 5 us (20 x 128 behind 6k-8k 330 -> 336, 14 x 128
+// it then cuts no tile, looking costs 3-6 us (20 x 128 behind 6k-8k 330 -> 336, 14 x 128
 // behind 4k 120 -> 125, 4 x 256 behind 4k 74 -> 78.5), so that it is done from 200 us on
 // with more tiles than slots, 100 with more than CUs and 60 with fewer.
 struct BalancedPlan {
